@@ -163,6 +163,27 @@ int ts_prefill_varlen(const void* q, const void* k_cache, const void* v_cache, v
                       int64_t bt_stride, float scale, int dtype, void* stream);
 
 /*
+ * ts_prefill_varlen with what a launch of few query tiles over long keys needs to cut them
+ * over more workgroups (prompt chunks behind a cached prefix): max_keys, an upper bound on
+ * every context length (the block table's width in keys), and a 16-byte aligned float32
+ * workspace of ts_prefill_workspace() floats, owned by this call until it has run. Without
+ * them (null, or fewer floats) it is ts_prefill_varlen. No reference counterpart.
+ */
+int ts_prefill_varlen_ws(const void* q, const void* k_cache, const void* v_cache, void* out,
+                         const int32_t* block_tables, const int32_t* q_starts,
+                         const int32_t* q_lens, const int32_t* context_lens, int R, int Hq,
+                         int Hkv, int D, int block_size, int max_q_len, int64_t n_rows,
+                         int64_t q_stride_t, int64_t q_stride_h, int64_t o_stride_t,
+                         int64_t o_stride_h, int64_t k_stride_slot, int64_t k_stride_head,
+                         int64_t bt_stride, float scale, int dtype, int64_t max_keys,
+                         float* workspace, int64_t workspace_floats, void* stream);
+
+/* Floats of workspace ts_prefill_varlen_ws uses for these sizes on the current device (0:
+ * it cuts nothing). */
+int64_t ts_prefill_workspace(int R, int Hq, int Hkv, int D, int block_size, int max_q_len,
+                             int64_t max_keys, int dtype);
+
+/*
  * RMSNorm of every row of x [T, N]:
  *   out = (T)(x * 1/sqrt(mean(x^2) + eps)) * w   (normalise in fp32, multiply in T)
  * Replaces _rms_norm_rows_kernel / rms_norm_rows (triton_fused.py:29-40, :116-126).

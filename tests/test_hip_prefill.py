@@ -17,6 +17,7 @@ from hypothesis import strategies as st
 
 from oracle import ref
 from tests.helpers import assert_contract, assert_matches
+from tinyserve_amd import hip_prefill
 from tinyserve_amd.hip_prefill import paged_prefill_attention
 from tinyserve_amd.workloads import PrefillCase, prefill_case, prefill_lengths
 
@@ -232,3 +233,41 @@ def test_length_ranked_sequence_groups(dtype: torch.dtype) -> None:
         out = torch.full_like(c.q, 7.0).to(DEVICE)
         run(c, out=out)
         check(c, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads", [(16, 8, 128), (32, 8, 128), (8, 2, 64), (8, 1, 128)])
+def test_long_keys_cut_over_workgroups(dtype: torch.dtype, heads: tuple[int, int, int]) -> None:
+    # Chunks behind long cached prefixes: few query tiles, so each one's key tiles are
+    # divided over several workgroups whose states are merged. One and 64 new tokens (the
+    # key-split shape), 65 and 128 (one 8-wave tile), 300 (several tiles, a partial one);
+    # lengths from one key to thousands in one launch (whole and cut items together, an
+    # empty sequence, prompts ending on and off a tile); parts whose first tile lies past
+    # some rows' positions.
+    hq, hkv, d = heads
+    cases = [([(3000, 1)], 16), ([(4000, 64), (0, 1), (700, 33)], 16), ([(1985, 65)], 32),
+             ([(40, 128), (3100, 100), (0, 128), (1000, 24)], 16)]  # fmt: skip
+    if hq // hkv <= 4:  # longer chunks at head groups of 8 keep whole items
+        cases.append(([(7000, 300)], 8))
+    for specs, bs in cases:
+        c = prefill_case(specs, hq, hkv, d, bs, dtype, seed=bs + len(specs), gap=1)
+        assert hip_prefill._workspace_floats(0, len(specs), hq, hkv, d, bs, c.max_q_len,
+                                             c.tables.shape[1] * bs, dtype) > 0  # fmt: skip
+        out = torch.full_like(c.q, 7.0).to(DEVICE)
+        run(c, out=out)
+        check(c, out)
+
+
+def test_cut_launch_replays_in_a_graph() -> None:
+    c = on_gpu(prefill_case([(2500, 90), (100, 20)], 16, 8, 128, 16, torch.float16, seed=5))
+    want = paged_prefill_attention(*c.args())
+    out = torch.empty_like(want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        paged_prefill_attention(*c.args(), out=out)
+    for _ in range(3):
+        out.fill_(9.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

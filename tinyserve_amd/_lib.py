@@ -51,6 +51,14 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _i64, _i64, _i64, _i64, _i64, _i64, _i64,  # strides
          _f, _i, _vp],
     ),
+    "ts_prefill_varlen_ws": (
+        _i,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,  # q k v out bt q_starts q_lens ctx_lens
+         _i, _i, _i, _i, _i, _i, _i64,  # R Hq Hkv D block_size max_q_len n_rows
+         _i64, _i64, _i64, _i64, _i64, _i64, _i64,  # strides
+         _f, _i, _i64, _vp, _i64, _vp],  # scale dtype max_keys workspace floats stream
+    ),
+    "ts_prefill_workspace": (_i64, [_i, _i, _i, _i, _i, _i, _i64, _i]),
     "ts_rms_norm_rows": (_i, [_vp, _vp, _vp, _i, _i, _i64, _i64, _f, _i, _vp]),
     "ts_qk_norm_rope_store": (
         _i,

@@ -29,6 +29,9 @@
 // deals workgroups to the 8 XCDs round-robin, with 8 kv heads each head's workgroups
 // share one XCD's L2, where its K/V blocks are re-read by every query tile.
 //
+// Few query tiles behind long cached prefixes are also cut along the keys over several
+// workgroups and merged by a second kernel (the key cut, below).
+//
 // Three shapes: 8 waves with a 3-stage ring of 64-key tiles (one workgroup per CU, 98 KB
 // of LDS, two waves per SIMD) for large launches and prefix-hit chunks; for launches with
 // too few query tiles to fill the chip that way (one or two prompts), 8 waves over the
@@ -110,9 +113,127 @@ struct PrefillArgs {
   int seq_group;  // > 0: dispatch in groups of this many sequences ranked by length
   int64_t q_st, q_sh, o_st, o_sh, k_ss, k_sh, bt_s;
   float scale_log2;
+  // Key cut (0 units: none): fp32 states of the cut items' parts, and the launch's units
+  // and CUs per (kv head, head chunk).
+  float* ws;
+  int32_t* ws_plan;  // [64][2]: each item's parts and first unit
+  int units;
+  int conc;
 };
 
 constexpr int kWin = 512;   // block ids held in LDS
+constexpr int kCutKeys = 64;  // keys per tile of the cut shapes
+
+// ---- key cut -----------------------------------------------------------------------------
+// A launch with fewer query tiles than CUs and long keys (prompt chunks behind a cached
+// prefix) waits for the workgroup with the longest walk while most of the chip idles. The
+// cut gives each item (sequence, query tile) several workgroups ("units") over near-equal
+// shares of its key tiles; cut items write fp32 softmax states (m, l, O^T) to the
+// workspace and prefill_merge_kernel merges them. The host knows sizes only, so every wave
+// derives the cut from the lengths itself: lane i holds item i's key tiles, lane j < 63
+// prices a share of about 4 x 1.12^j tiles and lane 63 whole items (written directly), and
+// the cheapest wins. In steps of one tile, on `conc` CUs: a unit costs its share plus
+// kCutUnit of start, end and state traffic; cutting at all costs kCutMerge, and kCutPart
+// per part of the longest item; all three are twice as many of the shorter steps of D = 64.
+constexpr float kWholeUnit = 2.0f, kCutUnit = 4.0f, kCutMerge = 4.0f, kCutPart = 0.25f;
+
+struct CutItem {
+  int item;   // r * n_qtiles + tile; -1: this unit has no work
+  int part;   // of `parts`
+  int parts;  // 1: whole
+  int tiles;  // key tiles per part (the last part may hold fewer)
+  int unit0;  // the item's first unit
+};
+
+// Key tiles of item i (0: no such query tile). BQ queries per tile.
+__device__ __forceinline__ int cut_tiles(const PrefillArgs& a, int i, int BQ) {
+  const int r = i / a.n_qtiles, tile = i - r * a.n_qtiles;
+  const int q_len = a.q_lens[r];
+  if (tile * BQ >= q_len) return 0;
+  const int keys = a.ctx_lens[r] - q_len + min((tile + 1) * BQ, q_len);
+  return (keys + kCutKeys - 1) / kCutKeys;
+}
+
+// Where every item's units lie: lane i gets item i's part count, tiles per part and first
+// unit (items <= 64; all lanes of the wave call).
+template <int D>
+__device__ __forceinline__ CutItem cut_plan(const PrefillArgs& a, int BQ) {
+  constexpr float kStep = 128.0f / D;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int items = a.R * a.n_qtiles;
+  const int t = lane < items ? cut_tiles(a, lane, BQ) : 0;
+  const float share = __builtin_floorf(4.0f * fast_exp2(static_cast<float>(lane) * 0.1635f));
+  const float inv = 1.0f / share;
+  float n = 0.f, total = 0.f, tmax = 1.f, live = 0.f;
+  for (int i = 0; i < items; ++i) {
+    const float ti = static_cast<float>(__builtin_amdgcn_readlane(t, i));
+    const float one = fminf(ti, 1.0f);
+    total += ti;
+    live += one;
+    tmax = fmaxf(tmax, ti);
+    n += fmaxf(__builtin_ceilf(ti * inv - 1e-3f), one);
+  }
+  const bool whole = lane == kWave - 1;
+  if (whole) n = live;
+  const float conc = static_cast<float>(a.conc);
+  // One round waits for its longest unit; several are balanced by the dispatch order but
+  // for about half a unit.
+  const float ps = whole ? tmax : fminf(share, tmax);
+  const float busy = n <= conc ? ps : fmaxf(ps, total / conc + 0.5f * ps);
+  float cost = busy + kStep * __builtin_ceilf(n / conc) * (whole ? kWholeUnit : kCutUnit);
+  if (!whole) cost += kStep * (kCutMerge + kCutPart * tmax * inv);
+  if (n > static_cast<float>(a.units)) cost = 3.0e6f;
+  // Cheapest share; ties to the larger one.
+  int key = static_cast<int>(fminf(cost, 3.0e6f) * 8.0f) * kWave + (kWave - 1 - lane);
+  for (int o = 1; o < kWave; o *= 2) key = min(key, __shfl_xor(key, o));
+  const int win = kWave - 1 - (__builtin_amdgcn_readfirstlane(key) & (kWave - 1));
+  const float win_inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), win));
+  CutItem c;
+  c.item = lane;
+  c.part = c.parts = c.tiles = c.unit0 = 0;
+  if (t > 0) {
+    c.parts = win == kWave - 1 ? 1 : max(static_cast<int>(__builtin_ceilf(static_cast<float>(t) * win_inv - 1e-3f)), 1);
+    c.tiles = (t + c.parts - 1) / c.parts;
+    c.parts = (t + c.tiles - 1) / c.tiles;  // no empty last part
+  }
+  // Units in order of falling size (ties by item), so that the longest start first.
+  const int size = c.tiles * kWave + (kWave - 1 - lane);
+  for (int i = 0; i < items; ++i)
+    c.unit0 += __builtin_amdgcn_readlane(size, i) > size ? __builtin_amdgcn_readlane(c.parts, i) : 0;
+  return c;
+}
+
+// The item and part that unit u works on (item -1: none), uniform over the wave. The
+// launch's first workgroup leaves every item's parts and first unit for the merge.
+template <int D>
+__device__ __forceinline__ CutItem cut_unit(const PrefillArgs& a, int BQ, int u) {
+  const CutItem p = cut_plan<D>(a, BQ);
+  if (blockIdx.x == 0 && threadIdx.x < kWave) {
+    a.ws_plan[2 * threadIdx.x] = p.parts;
+    a.ws_plan[2 * threadIdx.x + 1] = p.unit0;
+  }
+  const uint64_t hit = __ballot(p.parts > 0 && u >= p.unit0 && u < p.unit0 + p.parts);
+  CutItem c;
+  if (hit == 0) {
+    c.item = -1;
+    return c;
+  }
+  const int ln = __builtin_ctzll(hit);
+  c.item = ln;
+  c.parts = __builtin_amdgcn_readlane(p.parts, ln);
+  c.tiles = __builtin_amdgcn_readlane(p.tiles, ln);
+  c.unit0 = __builtin_amdgcn_readlane(p.unit0, ln);
+  c.part = u - c.unit0;
+  return c;
+}
+
+constexpr int kCutPlanFloats = 2 * kWave;  // the plan, at the workspace's start
+
+// Floats of one wave's state in the workspace: O^T [D / 32][4][64 lanes][4], m, l [64].
+template <int D>
+__host__ __device__ constexpr int64_t cut_state_floats() {
+  return static_cast<int64_t>(D / 2 + 2) * kWave;
+}
 
 template <int D, int W, int BN>
 struct TileShape {
@@ -188,7 +309,7 @@ __device__ __forceinline__ void ring_barrier() {
 }
 
 template <typename T, int D, int HG, int QB, int kWaves, int kStages, int kBN, int kOcc,
-          bool kScalarIds, int kParts>
+          bool kScalarIds, int kParts, bool kCut>
 __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(kOcc, kOcc))) void
 prefill_mfma_kernel(const PrefillArgs a) {
   using V8 = typename Mfma<T>::V8;
@@ -233,7 +354,13 @@ prefill_mfma_kernel(const PrefillArgs a) {
   const int rest = bid / n_hc;
   const int hcx = bid - rest * n_hc;
   int tile_rev, r;
-  if (a.seq_group > 0) {
+  CutItem cut;  // kCut: this workgroup's share of its item's key tiles
+  if constexpr (kCut) {
+    cut = cut_unit<D>(a, BQ, rest);
+    if (cut.item < 0) return;
+    r = cut.item / a.n_qtiles;
+    tile_rev = 0;
+  } else if (a.seq_group > 0) {
     // Groups of seq_group sequences of similar length, longest group first; within a
     // group, heaviest query tiles first. A group's K/V (one kv head per XCD) stays in
     // that XCD's L2 while its tiles run, which the plain order below loses when many
@@ -269,7 +396,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
     r = rest - tile_rev * a.R;
   }
   const int q_len = a.q_lens[r];
-  const int tile = (q_len + BQ - 1) / BQ - 1 - tile_rev;
+  const int tile = kCut ? cut.item - r * a.n_qtiles : (q_len + BQ - 1) / BQ - 1 - tile_rev;
   if (tile < 0) return;
   const int q0 = tile * BQ;
   const int ctx = a.ctx_lens[r];
@@ -285,7 +412,10 @@ prefill_mfma_kernel(const PrefillArgs a) {
   const int qi = wq0 + col;
   const bool q_ok = qi < q_len;
   const int pos = past + qi;
-  const int key_end = past + min(q0 + BQ, q_len);  // keys the workgroup needs
+  // Keys the workgroup needs: key_lo .. key_end - 1.
+  const int key_lo = kCut ? cut.part * cut.tiles * kBN : 0;
+  const int item_end = past + min(q0 + BQ, q_len);
+  const int key_end = kCut ? min(item_end, key_lo + cut.tiles * kBN) : item_end;
   const int key_last = key_end - 1;
   const int wave_key_end = wq0 < q_len ? past + min(wq0 + 32, q_len) : 0;
   const int wave_pos_min = past + wq0;
@@ -431,6 +561,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
   const int vd_lane = 16 * vdsub + 4 * (vj & 3);  // + 32 dt
   const int vswz = v_swz<D>(vkey_lane);           // key & 3 = vj >> 2 for every read
 
+  int first_key = 0;  // key of this wave's first tile
   auto attend = [&](const T* k_lds, const T* v_lds, int n0) __attribute__((always_inline)) {
     // S^T = K . Q^T for the tile's 32-key parts: NH independent MFMA chains. The K
     // operands of chunk kc + 1 are read while chunk kc multiplies.
@@ -514,8 +645,9 @@ prefill_mfma_kernel(const PrefillArgs a) {
     // exceeds 2^kRescale every P is at most 2^kRescale (exact in fp32, representable in
     // fp16/bf16) and the tile is done. Otherwise (whenever the scores grew by more than
     // kRescale) the exact maximum is taken, O and l are rescaled, and P is recomputed. A
-    // wave's first tile (n0 == 0 for every wave) starts from the exact maximum, so it
-    // needs no second pass: every row has a key there (key 0), so the maximum is finite.
+    // wave's first tile starts from the exact maximum, so it needs no second pass: at
+    // n0 == 0 every row has a key (key 0), so the maximum is finite; a cut part's first
+    // tile may mask a whole row, whose maximum then stays at m_run's finite start.
     auto tile_max = [&]() -> float {
       float mx = s[0][0];
 #pragma unroll
@@ -524,7 +656,11 @@ prefill_mfma_kernel(const PrefillArgs a) {
         for (int v = (h == 0 ? 1 : 0); v < 16; ++v) mx = fmaxf(mx, s[h][v]);
       return halves_max(mx) * c;
     };
-    if (n0 == 0) m_run = tile_max();
+    if constexpr (kCut) {
+      if (n0 == first_key) m_run = fmaxf(m_run, tile_max());
+    } else {
+      if (n0 == 0) m_run = tile_max();
+    }
     float psum = make_p();
     if (__any(!(psum <= exp2f(kRescale)))) {
       const float m_new = fmaxf(m_run, tile_max());
@@ -609,10 +745,11 @@ prefill_mfma_kernel(const PrefillArgs a) {
     // Part kh takes tiles kh * n_lo .. (kh + 1) * n_lo - 1 (the last part the rest); all
     // parts step n_lo times (the same barriers), later parts' last steps possibly with no
     // tile.
-    const int ntiles = (key_end + kBN - 1) / kBN;
+    const int ntiles = (key_end - key_lo + kBN - 1) / kBN;
     const int n_lo = (ntiles + kParts - 1) / kParts;
-    const int base = kh * n_lo * kBN;
-    const int half_end = kh == kParts - 1 ? key_end : min((kh + 1) * n_lo * kBN, key_end);
+    const int base = key_lo + kh * n_lo * kBN;
+    const int half_end = kh == kParts - 1 ? key_end : min(key_lo + (kh + 1) * n_lo * kBN, key_end);
+    first_key = base;
     auto sstep = [&](const T* k_cur, const T* v_cur, T* k_nx, T* v_nx, int n0) {
       ring_barrier<0>();
       if (n0 + kBN < half_end) gather(k_nx, v_nx, n0 + kBN);
@@ -625,23 +762,24 @@ prefill_mfma_kernel(const PrefillArgs a) {
       sstep(k1, v1, k0, v0, base + (i + 1) * kBN);
     }
   } else {
-  gather(k0, v0, 0);
-  if constexpr (kStages == 3) {
-    if (kBN < key_end) gather(k1, v1, kBN);
-    for (int n0 = 0; n0 < key_end; n0 += 3 * kBN) {
-      step(k0, v0, k2, v2, n0);
-      if (n0 + kBN >= key_end) break;
-      step(k1, v1, k0, v0, n0 + kBN);
-      if (n0 + 2 * kBN >= key_end) break;
-      step(k2, v2, k1, v1, n0 + 2 * kBN);
+    first_key = key_lo;
+    gather(k0, v0, key_lo);
+    if constexpr (kStages == 3) {
+      if (key_lo + kBN < key_end) gather(k1, v1, key_lo + kBN);
+      for (int n0 = key_lo; n0 < key_end; n0 += 3 * kBN) {
+        step(k0, v0, k2, v2, n0);
+        if (n0 + kBN >= key_end) break;
+        step(k1, v1, k0, v0, n0 + kBN);
+        if (n0 + 2 * kBN >= key_end) break;
+        step(k2, v2, k1, v1, n0 + 2 * kBN);
+      }
+    } else {
+      for (int n0 = key_lo; n0 < key_end; n0 += 2 * kBN) {
+        step(k0, v0, k1, v1, n0);
+        if (n0 + kBN >= key_end) break;
+        step(k1, v1, k0, v0, n0 + kBN);
+      }
     }
-  } else {
-    for (int n0 = 0; n0 < key_end; n0 += 2 * kBN) {
-      step(k0, v0, k1, v1, n0);
-      if (n0 + kBN >= key_end) break;
-      step(k1, v1, k0, v0, n0 + kBN);
-    }
-  }
   }
   // No load may still be writing this workgroup's LDS when its waves end.
   __builtin_amdgcn_s_waitcnt(0x0070);
@@ -688,6 +826,23 @@ prefill_mfma_kernel(const PrefillArgs a) {
   }
 
   const float l_tot = halves_sum(l_run);
+  if constexpr (kCut) {
+    if (cut.parts > 1) {
+      if (wq0 >= q_len) return;
+      float* st = a.ws + ((static_cast<int64_t>(rest) * n_hc + hcx) * kGW + wl) * cut_state_floats<D>();
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          typedef float F4 __attribute__((ext_vector_type(4)));
+          *reinterpret_cast<F4*>(st + ((dt * 4 + j) * kWave + lane) * 4) =
+              F4{oacc[dt][4 * j], oacc[dt][4 * j + 1], oacc[dt][4 * j + 2], oacc[dt][4 * j + 3]};
+        }
+      st[D / 2 * kWave + lane] = m_run;
+      st[(D / 2 + 1) * kWave + lane] = l_tot;
+      return;
+    }
+  }
   if (!q_ok) return;
   T* op = static_cast<T*>(a.out) + static_cast<int64_t>(q_start + qi) * a.o_st +
           static_cast<int64_t>(head) * a.o_sh;
@@ -704,6 +859,86 @@ prefill_mfma_kernel(const PrefillArgs a) {
     }
 }
 
+// Merges the parts of the cut items. One workgroup per (item, kv head and head chunk, wave
+// of 32 queries of one head); wave (pg, dt) takes 32 output dims of parts pg, pg + PG, ...:
+// it reads their m, then their l and O^T weighted by 2^(m - max m), and the PG groups merge
+// through LDS. Bound by the states' traffic (4 (D + 2) bytes per row and part, mostly still
+// in the last-level cache) or, with few items, by the round trips of one item's parts: PG
+// is 4 there. Whole items have been written by the main kernel.
+template <typename T, int D, int HG, int QB, int PG>
+__global__ __launch_bounds__(PG * D / 32 * kWave) void prefill_merge_kernel(const PrefillArgs a) {
+  constexpr int BQ = 32 * QB, GW = HG * QB, DT = D / 32;
+  typedef float F4 __attribute__((ext_vector_type(4)));
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  __shared__ float red[PG > 1 ? (PG - 1) * DT * 18 * kWave : 1];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int dt = wave % DT, pg = wave / DT;
+  const int n_hc = a.n_kvh * a.hchunks;
+  const int wl = blockIdx.x % GW;
+  const int hcx = blockIdx.x / GW % n_hc;
+  const int item = blockIdx.x / GW / n_hc;
+  const int parts = a.ws_plan[2 * item];
+  if (parts <= 1) return;
+  const int unit0 = a.ws_plan[2 * item + 1];
+  const int r = item / a.n_qtiles, tile = item - r * a.n_qtiles;
+  const int wq0 = tile * BQ + wl / HG * 32;
+  const int q_len = a.q_lens[r];
+  if (wq0 >= q_len) return;
+  const int64_t stride = static_cast<int64_t>(n_hc) * GW * cut_state_floats<D>();  // one unit
+  const float* st = a.ws + unit0 * stride + (static_cast<int64_t>(hcx) * GW + wl) * cut_state_floats<D>();
+  const float* ml = st + D / 2 * kWave + lane;
+  float m = -1.0e30f;
+#pragma unroll 8
+  for (int i = pg; i < parts; i += PG) m = fmaxf(m, ml[i * stride]);
+  float l = 0.f;
+  F4 acc[4] = {};
+#pragma unroll 4
+  for (int i = pg; i < parts; i += PG) {
+    const float w = fast_exp2(ml[i * stride] - m);
+    l += w * ml[i * stride + kWave];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc[j] += w * *reinterpret_cast<const F4*>(st + i * stride + ((dt * 4 + j) * kWave + lane) * 4);
+  }
+  if constexpr (PG > 1) {
+    auto slot = [&](int g) { return red + (g * DT + dt) * 18 * kWave + lane; };
+    if (pg > 0) {
+      float* x = slot(pg - 1);
+      x[0] = m;
+      x[kWave] = l;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) x[(2 + e) * kWave] = acc[e / 4][e % 4];
+    }
+    __syncthreads();
+    if (pg > 0) return;
+#pragma unroll
+    for (int g = 0; g < PG - 1; ++g) {
+      const float* x = slot(g);
+      const float mn = fmaxf(m, x[0]);
+      const float a0 = fast_exp2(m - mn), a1 = fast_exp2(x[0] - mn);
+      l = l * a0 + x[kWave] * a1;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e / 4][e % 4] = acc[e / 4][e % 4] * a0 + x[(2 + e) * kWave] * a1;
+      m = mn;
+    }
+  }
+  const int qi = wq0 + (lane & 31);
+  if (qi >= q_len) return;
+  const int kvh = hcx / a.hchunks;
+  const int head = kvh * a.group + (hcx - kvh * a.hchunks) * HG + wl % HG;
+  T* op = static_cast<T*>(a.out) + static_cast<int64_t>(a.q_starts[r] + qi) * a.o_st +
+          static_cast<int64_t>(head) * a.o_sh + dt * 32 + 4 * (lane >> 5);
+  const float inv = 1.f / l;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    T4 x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = static_cast<T>(acc[j][i] * inv);
+    *reinterpret_cast<T4*>(op + 8 * j) = x;
+  }
+}
+
 // KP > 1: the key-split shape (W waves, W / KP per key part); its caller checks that the
 // block size allows the scalar-id gather.
 template <typename T, int D, int HG, int W, int S, int BN, int OCC, int KP = 1>
@@ -712,14 +947,14 @@ static int launch_prefill_mfma(const PrefillArgs& a, int Hkv, hipStream_t stream
   const int seqs = a.seq_group > 0 ? (a.R + a.seq_group - 1) / a.seq_group * a.seq_group : a.R;
   dim3 grid(static_cast<unsigned>(a.n_qtiles) * seqs * Hkv * a.hchunks);
   if constexpr (KP > 1) {
-    hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, BN, OCC, true, KP>), grid,
+    hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, BN, OCC, true, KP, false>), grid,
                        dim3(W * kWave), 0, stream, a);
   } else {
     // A load's RPI rows share a cache block when blocks hold at least RPI slots.
     if ((1 << a.lbs) >= TileShape<D, W, BN>::kRPI)
-      hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, BN, OCC, true, 1>), grid, dim3(W * kWave), 0, stream, a);
+      hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, BN, OCC, true, 1, false>), grid, dim3(W * kWave), 0, stream, a);
     else
-      hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, BN, OCC, false, 1>), grid, dim3(W * kWave), 0, stream, a);
+      hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, BN, OCC, false, 1, false>), grid, dim3(W * kWave), 0, stream, a);
   }
   return launch_status();
 }
@@ -796,6 +1031,92 @@ static PrefillShape prefill_shape(int R, int group, int Hkv, int max_q_len, int6
   return PrefillShape::kW8;
 }
 
+// ---- the key cut's launches --------------------------------------------------------------
+// Its two shapes, both over 64-key tiles: up to 64 new tokens per sequence the key-split
+// one (64 queries x 2 heads, two key halves inside the workgroup), else the 8-wave one.
+struct CutShape {
+  int hg, waves;  // heads per workgroup; waves over the queries and heads
+  int n_qtiles, hchunks, units, conc;
+};
+
+// Whether a launch of these sizes may cut its keys, and how. max_keys: the block table's
+// width in keys, the most any sequence can have. The line: what a cut can save must exceed
+// the plan (~1 us), the merge launch (2 us empty, 9-10 us with 2-4 parts of 100 rows x 16
+// sequences) and the states' traffic. Measured at 16 q / 8 kv heads, D = 128, fp16 (cached
+// + new tokens, uncut -> cut, us): 16 x (500-5000 + 20-128) 114 -> 60, 1 x (8192 + 64)
+// 109 -> 26, 1 x (8192 + 512) 111 -> 55, 1 x (16000 + 32) 203 -> 29, 6 x (3000 + 128)
+// 79 -> 42, 24 x (0-6000 + 10-128) 144 -> 96, 8 x (2000 + 16) 32 -> 25; with equal lengths
+// on most of the chip the plan keeps items whole and costs 2-3 us (24 x (4096 + 128)
+// 136 -> 139). Below the line it lost: 4 x (1024 + 64) 21 -> 26, 4 x (8192 + 300) 115 ->
+// 125, 1 x (1500 + 256) 29 -> 33, 16 x (4096 + 64) 73 -> 75, 32 x (2048 + 128) 94 -> 99.
+static bool cut_shape(int R, int group, int Hkv, int D, int lbs, int max_q_len, int64_t max_keys, CutShape* c) {
+  if (max_q_len > 512 || max_keys < 1024 || max_keys < 4 * static_cast<int64_t>(max_q_len)) return false;
+  if ((1 << lbs) < kWave / (D / 8)) return false;  // scalar-id gather
+  c->waves = max_q_len <= 64 && group <= 4 ? 4 : 8;
+  c->hg = group < c->waves ? group : c->waves;
+  c->hchunks = group / c->hg;
+  const int bq = 32 * (c->waves / c->hg);
+  c->n_qtiles = (max_q_len + bq - 1) / bq;
+  const int n_hc = Hkv * c->hchunks;
+  const int64_t items = static_cast<int64_t>(R) * c->n_qtiles;
+  const int cus = compute_units();
+  if (items > kWave) return false;
+  // What a cut can gain, in steps of the longest workgroup of the shape that runs
+  // otherwise (`fill`: its workgroups per CU).
+  const bool halves = prefill_shape(R, group, Hkv, max_q_len, 0) == PrefillShape::kW4;
+  if (!halves && max_q_len > 128) return false;
+  const int hg = halves ? std::min(group, 4) : std::min(group, 8);
+  const int oq = 32 * ((halves ? 4 : 8) / hg);
+  const double fill = static_cast<double>((max_q_len + oq - 1) / oq) * R * Hkv * (group / hg) / cus;
+  const double steps = static_cast<double>(max_keys) / (halves ? 2 * kCutKeys : kCutKeys);
+  const double gain = steps * (1.0 - (halves ? 1.6 : 1.0) * fill);
+  if (gain < (halves && (max_q_len > 128 || D == 64) ? 20.0 : 9.0 * (128 / D))) return false;
+  c->conc = cus / n_hc > 1 ? cus / n_hc : 1;
+  c->units = static_cast<int>(std::max<int64_t>(items, 2 * c->conc));
+  return true;
+}
+
+template <typename T, int D, int HG, int W, int S, int KP>
+static int launch_cut(const PrefillArgs& a, hipStream_t stream) {
+  constexpr int GW = W / KP, QB = GW / HG;
+  const int n_hc = a.n_kvh * a.hchunks;
+  hipLaunchKernelGGL((prefill_mfma_kernel<T, D, HG, QB, W, S, kCutKeys, 2, true, KP, true>), dim3(a.units * n_hc),
+                     dim3(W * kWave), 0, stream, a);
+  if (const int rc = launch_status()) return rc;
+  const int items = a.R * a.n_qtiles;
+  if (items <= 8)
+    hipLaunchKernelGGL((prefill_merge_kernel<T, D, HG, QB, 4>), dim3(items * n_hc * GW), dim3(4 * D / 32 * kWave), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((prefill_merge_kernel<T, D, HG, QB, 1>), dim3(items * n_hc * GW), dim3(D / 32 * kWave), 0,
+                       stream, a);
+  return launch_status();
+}
+
+template <typename T, int D>
+static int dispatch_cut(PrefillArgs& a, const CutShape& c, int Hkv, hipStream_t stream) {
+  a.hchunks = c.hchunks;
+  a.n_qtiles = c.n_qtiles;
+  a.n_kvh = Hkv;
+  a.seq_group = 0;
+  a.units = c.units;
+  a.conc = c.conc;
+  a.ws += kCutPlanFloats;  // the plan comes first
+  if (c.waves == 4) {
+    switch (c.hg) {
+      case 1: return launch_cut<T, D, 1, 8, 2, 2>(a, stream);
+      case 2: return launch_cut<T, D, 2, 8, 2, 2>(a, stream);
+      default: return launch_cut<T, D, 4, 8, 2, 2>(a, stream);
+    }
+  }
+  switch (c.hg) {
+    case 1: return launch_cut<T, D, 1, 8, 3, 1>(a, stream);
+    case 2: return launch_cut<T, D, 2, 8, 3, 1>(a, stream);
+    case 4: return launch_cut<T, D, 4, 8, 3, 1>(a, stream);
+    default: return launch_cut<T, D, 8, 8, 3, 1>(a, stream);
+  }
+}
+
 template <typename T, int D>
 static int dispatch_hg(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows, hipStream_t stream) {
   switch (prefill_shape(a.R, a.group, Hkv, max_q_len, n_rows)) {
@@ -821,6 +1142,25 @@ int prefill_rows_generic(const void* q, const void* k, const void* v, void* out,
 
 using namespace ts;
 
+// Whether the MFMA kernels take these types and rows: their direct-to-LDS gather moves
+// 16-byte units, so rows must start 16-byte aligned.
+static bool mfma_rows(const void* k, const void* v, int64_t k_ss, int64_t k_sh, int D, int dtype) {
+  return (dtype == TS_F16 || dtype == TS_BF16) && (D == 64 || D == 128) && k_ss % 8 == 0 && k_sh % 8 == 0 &&
+         reinterpret_cast<uintptr_t>(k) % 16 == 0 && reinterpret_cast<uintptr_t>(v) % 16 == 0;
+}
+
+extern "C" int64_t ts_prefill_workspace(int R, int Hq, int Hkv, int D, int block_size, int max_q_len,
+                                        int64_t max_keys, int dtype) {
+  if (R <= 0 || max_q_len <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || !is_pow2(Hq / Hkv) || !is_pow2(block_size))
+    return 0;
+  CutShape c;
+  if ((dtype != TS_F16 && dtype != TS_BF16) || (D != 64 && D != 128) ||
+      !cut_shape(R, Hq / Hkv, Hkv, D, ilog2(block_size), max_q_len, max_keys, &c))
+    return 0;
+  return kCutPlanFloats + static_cast<int64_t>(c.units) * Hkv * c.hchunks * c.waves *
+         (D == 128 ? cut_state_floats<128>() : cut_state_floats<64>());
+}
+
 extern "C" int ts_prefill_varlen(const void* q, const void* k_cache, const void* v_cache,
                                  void* out, const int32_t* block_tables,
                                  const int32_t* q_starts, const int32_t* q_lens,
@@ -830,20 +1170,36 @@ extern "C" int ts_prefill_varlen(const void* q, const void* k_cache, const void*
                                  int64_t q_stride_h, int64_t o_stride_t, int64_t o_stride_h,
                                  int64_t k_stride_slot, int64_t k_stride_head,
                                  int64_t bt_stride, float scale, int dtype, void* stream) {
+  return ts_prefill_varlen_ws(q, k_cache, v_cache, out, block_tables, q_starts, q_lens, context_lens, R, Hq, Hkv, D,
+                              block_size, max_q_len, n_rows, q_stride_t, q_stride_h, o_stride_t, o_stride_h,
+                              k_stride_slot, k_stride_head, bt_stride, scale, dtype, 0, nullptr, 0, stream);
+}
+
+extern "C" int ts_prefill_varlen_ws(const void* q, const void* k_cache, const void* v_cache, void* out,
+                                    const int32_t* block_tables, const int32_t* q_starts, const int32_t* q_lens,
+                                    const int32_t* context_lens, int R, int Hq, int Hkv, int D, int block_size,
+                                    int max_q_len, int64_t n_rows, int64_t q_stride_t, int64_t q_stride_h,
+                                    int64_t o_stride_t, int64_t o_stride_h, int64_t k_stride_slot,
+                                    int64_t k_stride_head, int64_t bt_stride, float scale, int dtype,
+                                    int64_t max_keys, float* workspace, int64_t workspace_floats, void* stream) {
   if (R < 0 || max_q_len < 0 || n_rows < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || !is_pow2(Hq / Hkv) ||
       !is_pow2(block_size))
     return TS_EINVAL;
   if (R == 0 || max_q_len == 0) return 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int lbs = ilog2(block_size);
-  // The direct-to-LDS gather moves 16-byte units: rows must start 16-byte aligned.
-  const bool aligned = (k_stride_slot % 8 == 0) && (k_stride_head % 8 == 0) &&
-                       (reinterpret_cast<uintptr_t>(k_cache) % 16 == 0) &&
-                       (reinterpret_cast<uintptr_t>(v_cache) % 16 == 0);
-  if ((dtype == TS_F16 || dtype == TS_BF16) && (D == 64 || D == 128) && aligned) {
+  if (mfma_rows(k_cache, v_cache, k_stride_slot, k_stride_head, D, dtype)) {
     PrefillArgs a{q, k_cache, v_cache, out, block_tables, q_starts, q_lens, context_lens,
                   R, Hq / Hkv, 1, lbs, 1, Hkv, 0, q_stride_t, q_stride_h, o_stride_t, o_stride_h,
-                  k_stride_slot, k_stride_head, bt_stride, scale * kLog2e};
+                  k_stride_slot, k_stride_head, bt_stride, scale * kLog2e, workspace, reinterpret_cast<int32_t*>(workspace), 0, 0};
+    CutShape c;
+    const int64_t need = workspace ? ts_prefill_workspace(R, Hq, Hkv, D, block_size, max_q_len, max_keys, dtype) : 0;
+    if (need > 0 && workspace_floats >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
+        cut_shape(R, Hq / Hkv, Hkv, D, lbs, max_q_len, max_keys, &c)) {
+      if (dtype == TS_F16)
+        return D == 64 ? dispatch_cut<f16, 64>(a, c, Hkv, st) : dispatch_cut<f16, 128>(a, c, Hkv, st);
+      return D == 64 ? dispatch_cut<bf16, 64>(a, c, Hkv, st) : dispatch_cut<bf16, 128>(a, c, Hkv, st);
+    }
     if (dtype == TS_F16) {
       return D == 64 ? dispatch_hg<f16, 64>(a, Hkv, max_q_len, n_rows, st)
                      : dispatch_hg<f16, 128>(a, Hkv, max_q_len, n_rows, st);

@@ -18,6 +18,8 @@ and other head dims run the decode kernel's loop, one wave per (query row, kv he
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from tinyserve_amd import _lib
@@ -25,6 +27,14 @@ from tinyserve_amd import _lib
 # The reference's Triton tile (rows_per_tile, block_n, num_warps), :47. The arguments are
 # validated as the reference does and otherwise unused: the HIP kernels choose their tiles.
 DEFAULT_TILE = (64, 32, 8)
+
+
+@functools.lru_cache(maxsize=4096)
+def _workspace_floats(device: int, r: int, hq: int, hkv: int, d: int, block_size: int, max_q_len: int,
+                      max_keys: int, dtype: torch.dtype) -> int:  # fmt: skip
+    """Floats of workspace a launch of these sizes uses on ``device`` (which sets the CU
+    count) to cut long keys over more workgroups; 0 if it does not cut them."""
+    return _lib.load().ts_prefill_workspace(r, hq, hkv, d, block_size, max_q_len, max_keys, _lib.DTYPES[dtype])
 
 
 def paged_prefill_attention(
@@ -104,13 +114,17 @@ def paged_prefill_attention(
     if r == 0 or t == 0:
         return out
     dev = _lib.require_device(q, k_cache, v_cache, block_tables, q_starts, q_lens, context_lens, out)
+    max_q_len = int(max_q_len)
+    max_keys = block_tables.shape[1] * block_size
+    floats = _workspace_floats(dev, r, num_q_heads, num_kv_heads, head_dim, block_size, max_q_len, max_keys, q.dtype)
+    ws = torch.empty(floats, dtype=torch.float32, device=q.device) if floats else None
     _lib.call(
-        "ts_prefill_varlen",
+        "ts_prefill_varlen_ws",
         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
         block_tables.data_ptr(), q_starts.data_ptr(), q_lens.data_ptr(), context_lens.data_ptr(),
-        r, num_q_heads, num_kv_heads, head_dim, block_size, int(max_q_len), t,
+        r, num_q_heads, num_kv_heads, head_dim, block_size, max_q_len, t,
         q.stride(0), q.stride(1), out.stride(0), out.stride(1),
         k_cache.stride(0), k_cache.stride(1), block_tables.stride(0),
-        float(scale), _lib.dtype_code(q), _lib.stream_of(dev),
+        float(scale), _lib.dtype_code(q), max_keys, _lib.ptr(ws), floats, _lib.stream_of(dev),
     )  # fmt: skip
     return out
