@@ -238,3 +238,23 @@ def test_add_rms_norm_random_widths_and_partial_counts(seed: int) -> None:
     assert torch.equal(x, want_x)
     dense = h.to_dense() if seed % 2 else h
     assert torch.equal(dense, rms_norm_rows(want_x, w, EPS))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 31, 32, 33])
+@pytest.mark.parametrize(("n", "k"), [(1024, 1024), (96, 96)])
+def test_few_rows_equal_the_same_rows_of_a_full_block(m: int, n: int, k: int, dtype: torch.dtype) -> None:
+    # At most 16 and 32 rows run one and two of a row block's four 16-row tiles; the sums
+    # and their order are those of the whole block, so the rows match bit for bit.
+    x, w = operands(64, 2 * n, k, dtype, seed=4)
+    half = w[:n]
+    for few, full in ((x[:m], x), (Tiled.from_dense(x[:m].contiguous()), Tiled.from_dense(x))):
+        assert torch.equal(rows_linear(few, half), rows_linear(full, half)[:m])
+        part, ks = rows_linear_partials(few, half)
+        want, full_ks = rows_linear_partials(full, half)
+        assert ks == full_ks and torch.equal(part, want[:, :m])
+        act, want = rows_silu_gate_up(few, w), rows_silu_gate_up(full, w)
+        assert torch.equal(act.to_dense(), want.to_dense()[:m])
+        padded = Tiled(act.buf, 64, n).to_dense()
+        assert not padded[m:].any()

@@ -90,13 +90,21 @@ struct RowsArgs {
 
 // Lane l of a 16 x 32 operand holds row l % 16 and columns 8 (l / 16) .. + 7; the 16 x 16
 // fp32 result holds column l % 16 (a row of x) and rows 4 (l / 16) .. + 3 (rows of W).
-template <typename T, int KP, int NTW, int STEPS, bool XT, int EPI>
+//
+// MT: 16-row tiles of x a workgroup multiplies (4, or fewer when the launch has at most 16
+// or 32 rows). x is re-read by every workgroup, so at few rows its loads, not W's, are most
+// of the traffic: the unused tiles of a 64-row block are neither loaded nor multiplied.
+// Measured as below, all four tiles -> the tiles that hold rows (us): 32 rows, qkv 5.6 ->
+// 4.7, o_proj 4.0 -> 3.7, gate_up 7.4 -> 6.3, down 4.7 -> 4.2; one row, 5.5 -> 4.1, 3.6 ->
+// 3.2, 7.2 -> 5.5, 4.7 -> 3.9.
+template <typename T, int KP, int NTW, int STEPS, int MT, bool XT, int EPI>
 __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a) {
   using V8 = typename Mfma16x32<T>::V8;
   static_assert(EPI != kSiluGateUp || NTW == 2, "SiLU epilogue: one gate and one up tile per wave");
   constexpr int BN = 16 * NTW;  // W rows per workgroup
   constexpr int RED = BN + 1;   // padded row of the part sums
-  __shared__ float red[KP > 1 ? KP * kRowBlock * RED : 1];
+  constexpr int ROWS = 16 * MT;  // rows of x per workgroup
+  __shared__ float red[KP > 1 ? KP * ROWS * RED : 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -118,19 +126,19 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
   };
   // x row of MFMA tile mt for this lane (rows past M read row M - 1: finite, never
   // stored).
-  int xrow[4];
+  int xrow[MT];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) xrow[mt] = min(mb * kRowBlock + mt * 16 + r16, a.M - 1);
+  for (int mt = 0; mt < MT; ++mt) xrow[mt] = min(mb * kRowBlock + mt * 16 + r16, a.M - 1);
 
-  r_f32x4 acc[NTW][4];
+  r_f32x4 acc[NTW][MT];
 #pragma unroll
   for (int t = 0; t < NTW; ++t)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[t][mt] = r_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = r_f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (int c = 0; c < a.kchunks; ++c) {
     const int k0 = (blockIdx.z * a.kchunks + c) * CH + kp * (STEPS * 32);  // this wave's columns
-    V8 wv[STEPS][NTW], xv[STEPS][4];
+    V8 wv[STEPS][NTW], xv[STEPS][MT];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
       const int k = k0 + s * 32;
@@ -138,7 +146,7 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
       for (int t = 0; t < NTW; ++t)
         wv[s][t] = *reinterpret_cast<const V8*>(wg + static_cast<int64_t>(w_row(t)) * a.ws + k + kq);
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
+      for (int mt = 0; mt < MT; ++mt) {
         if constexpr (XT) {
           const int64_t unit = (static_cast<int64_t>(mb) * (a.K / 32) + k / 32) * 4 + mt;
           xv[s][mt] = *reinterpret_cast<const V8*>(xg + unit * 512 + lane * 8);
@@ -154,7 +162,7 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
 #pragma unroll
       for (int t = 0; t < NTW; ++t)
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) acc[t][mt] = Mfma16x32<T>::mma(wv[s][t], xv[s][mt], acc[t][mt]);
+        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = Mfma16x32<T>::mma(wv[s][t], xv[s][mt], acc[t][mt]);
   }
 
   // Sum of the KP waves' parts of element (m, j), j < BN the workgroup's W row.
@@ -162,16 +170,16 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          red[(kp * kRowBlock + mt * 16 + r16) * RED + t * 16 + (lane >> 4) * 4 + i] = acc[t][mt][i];
+          red[(kp * ROWS + mt * 16 + r16) * RED + t * 16 + (lane >> 4) * 4 + i] = acc[t][mt][i];
     __syncthreads();
   }
   auto total = [&](int m, int j) {
     float v = 0.f;
 #pragma unroll
-    for (int p = 0; p < KP; ++p) v += red[(p * kRowBlock + m) * RED + j];
+    for (int p = 0; p < KP; ++p) v += red[(p * ROWS + m) * RED + j];
     return v;
   };
 
@@ -193,7 +201,7 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
   } else if constexpr (KP > 1) {
     // Thread u handles 8 consecutive columns of one row: 16-byte stores.
     constexpr int GROUPS = BN / 8;
-    for (int u = tid; u < kRowBlock * GROUPS; u += KP * kWave) {
+    for (int u = tid; u < ROWS * GROUPS; u += KP * kWave) {
       const int m = u / GROUPS, j0 = (u % GROUPS) * 8;
       const int row = mb * kRowBlock + m;
       if (row >= a.M) continue;
@@ -219,9 +227,9 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float v = 0.f;  // rows past M: zeros (the tiled output is read whole)
-          if (row < a.M) {
-            const float g = to_f32(from_f32<T>(acc[0][mt][i]));
-            const float up = to_f32(from_f32<T>(acc[1][mt][i]));
+          if (mt < MT && row < a.M) {
+            const float g = to_f32(from_f32<T>(acc[0][mt < MT ? mt : 0][i]));
+            const float up = to_f32(from_f32<T>(acc[1][mt < MT ? mt : 0][i]));
             v = to_f32(from_f32<T>(g / (1.0f + expf(-g)))) * up;
           }
           static_cast<T*>(a.out)[tiled_index(row, n0 + (lane >> 4) * 4 + i, a.N)] = from_f32<T>(v);
@@ -232,7 +240,7 @@ __global__ __launch_bounds__(KP * kWave) void rows_gemm_kernel(const RowsArgs a)
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
+      for (int mt = 0; mt < MT; ++mt) {
         const int row = mb * kRowBlock + mt * 16 + r16;
         if (row >= a.M) continue;
 #pragma unroll
@@ -306,19 +314,26 @@ static bool plan_rows(int M, int N, int K, int epi, RowsPlan* p) {
   return found;
 }
 
-template <typename T, int KP, int NTW, int STEPS, int EPI>
+template <typename T, int KP, int NTW, int STEPS, int MT, int EPI>
 static int launch_rows(const RowsArgs& a, bool xt, hipStream_t st) {
   const int bn = EPI == kSiluGateUp ? 16 : 16 * NTW;
-  const dim3 grid(a.N / bn, (a.M + kRowBlock - 1) / kRowBlock, a.ks);
-  if (xt) hipLaunchKernelGGL((rows_gemm_kernel<T, KP, NTW, STEPS, true, EPI>), grid, dim3(KP * kWave), 0, st, a);
-  else hipLaunchKernelGGL((rows_gemm_kernel<T, KP, NTW, STEPS, false, EPI>), grid, dim3(KP * kWave), 0, st, a);
+  const dim3 grid(a.N / bn, (a.M + kRowBlock - 1) / kRowBlock, a.ks), block(KP * kWave);
+  if (xt) hipLaunchKernelGGL((rows_gemm_kernel<T, KP, NTW, STEPS, MT, true, EPI>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((rows_gemm_kernel<T, KP, NTW, STEPS, MT, false, EPI>), grid, block, 0, st, a);
   return launch_status();
+}
+
+template <typename T, int KP, int NTW, int STEPS, int EPI>
+static int launch_rows_mt(const RowsArgs& a, bool xt, hipStream_t st) {
+  if (a.M <= 16) return launch_rows<T, KP, NTW, STEPS, 1, EPI>(a, xt, st);
+  if (a.M <= 32) return launch_rows<T, KP, NTW, STEPS, 2, EPI>(a, xt, st);
+  return launch_rows<T, KP, NTW, STEPS, 4, EPI>(a, xt, st);
 }
 
 template <typename T, int EPI>
 static int dispatch_rows(const RowsArgs& a, const RowsPlan& p, bool xt, hipStream_t st) {
 #define TS_ROWS(KP, NTW, S)                                      \
-  if (p.kp == KP && p.ntw == NTW && p.steps == S) return launch_rows<T, KP, NTW, S, EPI>(a, xt, st);
+  if (p.kp == KP && p.ntw == NTW && p.steps == S) return launch_rows_mt<T, KP, NTW, S, EPI>(a, xt, st);
   if constexpr (EPI == kStore) {
     TS_ROWS(8, 1, 4) TS_ROWS(8, 1, 2) TS_ROWS(4, 1, 2) TS_ROWS(4, 1, 1) TS_ROWS(2, 1, 1) TS_ROWS(1, 1, 1)
   } else if constexpr (EPI == kPartial) {
