@@ -160,6 +160,14 @@ def test_policy_splits_for_small_grids(lib: ctypes.CDLL) -> None:
     assert policy(16, 128) == 1  # half the chip: one launch
 
 
+def test_policy_runs_short_tables_as_one_launch(lib: ctypes.CDLL) -> None:
+    # Small grids over short tables: 512 tokens x heads per wave, both sides of the line,
+    # for one, two and four (of eight) heads a wave.
+    for hq, line in ((8, 32), (16, 16), (32, 8), (64, 8)):
+        assert hip_attention.policy_splits(4, hq, 8, 128, 16, line) == 1
+        assert hip_attention.policy_splits(4, hq, 8, 128, 16, line + 1) > 1
+
+
 # --- decode entry points: the reference's argument errors (test_triton_attention.py:201-234)
 
 

@@ -65,6 +65,15 @@ IN_GROUP_SPLITS = 4
 # writing fp32 partials, then the combine, finish sooner.
 IN_GROUP_MIN_WAVES = 1024
 
+# Tables of at most this many tokens x query heads per wave run as one launch whatever the
+# grid: the workgroup's waves walk a few dozen tokens each, and partials would add a second
+# launch and its round trip. Measured (graph replay, B = 1 to 8, one launch against the
+# policy's partials, us): 16 q / 8 kv heads fp16 208 tokens 6.9 against 7.6-8.4, 256 tokens
+# 6.9 against 7.8-8.4, fp32 256 tokens 7.7 against 8.2-8.6; 32 / 8 heads (four per wave) 128
+# tokens 7.8 against 9.1-10.1 but 208 tokens 10.8 against 9.2-11.0; called eagerly, 8.5-9.2
+# against 18-19 (two launches and three allocations of host time).
+ONE_LAUNCH_TOKEN_HEADS = 512
+
 # Reference constants, kept for ``num_splits_for(..., target=..., no_split=...)`` callers
 # that want the T4 policy exactly.
 T4_TARGET_PROGRAMS = 1024
@@ -177,11 +186,15 @@ def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int
     and a count up to ``IN_GROUP_SPLITS`` becomes one launch whose workgroups split each
     sequence over their waves. A smaller grid gets enough split ranges for about twice
     the chip (at most ``MAX_SPLITS`` and the table width), as fp32 partials and the
-    combine. Sizes only (``device`` sets the CU count): a graph-captured launch keeps its
+    combine, unless its tables are so short (``ONE_LAUNCH_TOKEN_HEADS``) that one launch is
+    faster. Sizes only (``device`` sets the CU count): a graph-captured launch keeps its
     grid."""
     splits = num_splits_for(batch, num_kv_heads, max_blocks)
     simds = _one_split_waves(device, batch, num_q_heads, num_kv_heads, head_dim, block_size,
                              max_blocks, dtype)  # fmt: skip
+    heads = min(num_q_heads // num_kv_heads, 4)  # per wave
+    if head_dim <= 128 and max_blocks * block_size * heads <= ONE_LAUNCH_TOKEN_HEADS:
+        return 1
     if simds >= IN_GROUP_MIN_WAVES // 2:
         return 1 if splits <= IN_GROUP_SPLITS else splits
     return max(splits, min(-(-2 * IN_GROUP_MIN_WAVES // max(simds, 1)), MAX_SPLITS, max_blocks))
