@@ -202,6 +202,23 @@ int ts_rope_cos_sin(const int64_t* positions, int T, int D, double theta, float*
                     float* sin_out, int64_t stride, void* stream);
 
 /*
+ * x = round(x + y) in place, then out = RMSNorm(x) * w as ts_rms_norm_rows (the residual add
+ * and norm of the decoder layer, reference src/tinyserve/model.py:172-179). Rows of up to 4096
+ * 16-bit or 2048 32-bit elements, 16-byte aligned; others return TS_EUNSUPPORTED.
+ */
+int ts_add_rms_norm_rows(void* x, const void* y, const void* w, void* out, int T, int N,
+                         int64_t x_stride, int64_t y_stride, int64_t o_stride, float eps,
+                         int dtype, void* stream);
+
+/*
+ * act[t] = silu(gate_up[t][:N]) * gate_up[t][N:2N], each rounded to the type (reference
+ * src/tinyserve/model.py:176-178). Rows 16-byte aligned, N a multiple of 16 bytes; others
+ * return TS_EUNSUPPORTED.
+ */
+int ts_silu_mul(const void* gate_up, void* act, int T, int N, int64_t g_stride,
+                int64_t a_stride, int dtype, void* stream);
+
+/*
  * Per-head RMSNorm + rotate-half RoPE of q and k, and the paged KV-cache write.
  * Replaces _qk_norm_rope_store_kernel / qk_norm_rope_store (triton_fused.py:43-113,
  * :129-177).

@@ -14,7 +14,7 @@ import torch
 
 from oracle import ref
 from tests.helpers import ULP, assert_contract, assert_matches
-from tinyserve_amd.hip_fused import qk_norm_rope_store, rms_norm_rows, rope_cos_sin
+from tinyserve_amd.hip_fused import add_rms_norm_rows, qk_norm_rope_store, rms_norm_rows, rope_cos_sin, silu_mul
 from tinyserve_amd.workloads import fused_case
 
 pytestmark = pytest.mark.gpu
@@ -175,3 +175,35 @@ def test_rope_cos_sin_rejects_bad_arguments() -> None:
         rope_cos_sin(63, 1e6, torch.arange(4, device=DEVICE))
     c, s = rope_cos_sin(64, 1e6, torch.empty(0, dtype=torch.int64, device=DEVICE))
     assert c.shape == s.shape == (0, 64)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize(("t", "n"), [(1, 8), (3, 1024), (1023, 520), (1025, 1024), (700, 4096), (5, 6000), (4, 37)])
+def test_add_rms_norm_rows_is_the_add_then_the_norm(t: int, n: int, dtype: torch.dtype) -> None:
+    # Rows per workgroup on both sides of the line (4 per CU), widths that fill and part-fill
+    # a wave's chunks, and rows that take the two launches (too long, unaligned).
+    g = torch.Generator().manual_seed(t + n)
+    x, y, w = (torch.randn(*s, generator=g).to(DEVICE, dtype) for s in ((t, n), (t, n), (n,)))
+    want_x = x + y
+    want = rms_norm_rows(want_x, w, 1e-6)
+    got = add_rms_norm_rows(x, y, w, 1e-6)
+    assert torch.equal(x, want_x) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize(("t", "n"), [(1, 8), (7, 24), (333, 3072), (2, 5)])
+def test_silu_mul_equals_torch(t: int, n: int, dtype: torch.dtype) -> None:
+    # Against the same ops in float64 with their roundings: SiLU rounded, then the product.
+    # The fp32 SiLU may round to the other neighbour of a near-tie: one ulp of the SiLU
+    # carried to the product, and the product's own half ulp.
+    g = torch.Generator().manual_seed(n)
+    gu = (torch.randn(t, 2 * n, generator=g) * 4).to(DEVICE, dtype)
+    gu[0, 0], gu[0, n] = -200.0, 1.5  # exp(200) is infinite in fp32: silu is -0
+    gate, up = gu.double().chunk(2, dim=1)
+    silu = torch.nn.functional.silu(gate).to(dtype).double()
+    want = (silu * up).to(dtype)
+    got = silu_mul(gu)
+    assert torch.isfinite(got).all()
+    ulp = {torch.float32: 2.0**-22, torch.float16: 2.0**-10, torch.bfloat16: 2.0**-7}[dtype]
+    tiny = {torch.float32: 1e-30, torch.float16: 2.0**-23, torch.bfloat16: 1e-30}[dtype]
+    assert ((got.double() - want.double()).abs() <= 2 * ulp * want.double().abs() + tiny * (1 + up.abs())).all()

@@ -60,6 +60,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "ts_prefill_workspace": (_i64, [_i, _i, _i, _i, _i, _i, _i64, _i]),
     "ts_rms_norm_rows": (_i, [_vp, _vp, _vp, _i, _i, _i64, _i64, _f, _i, _vp]),
+    "ts_add_rms_norm_rows": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i64, _i64, _i64, _f, _i, _vp]),
+    "ts_silu_mul": (_i, [_vp, _vp, _i, _i, _i64, _i64, _i, _vp]),
     "ts_qk_norm_rope_store": (
         _i,
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,  # tensors

@@ -20,8 +20,9 @@ then the final norm (adding the last layer's down partials) and the tied output 
 (model.py:214-221). Other dtypes and larger row counts (a mixed prefill step) take the
 projections through library GEMMs instead:
 
-    h = rms_norm_rows(x); qkv = h @ W_qkv^T; ...; x += attn @ W_o^T (rounded, then added in place);
-    h = rms_norm_rows(x); x += (silu(gate) * up) @ W_down^T
+    h = add_rms_norm_rows(x, previous layer's down product); qkv = h @ W_qkv^T; ...
+    h = add_rms_norm_rows(x, attn @ W_o^T)          (rounded, then added in place)
+    down = silu_mul(h @ W_gate_up^T) @ W_down^T     (added by the next norm)
 
 Weights are random (no checkpoints here): linear weights ~ N(0, 0.02) in the model dtype,
 norm weights 1 + 0.1 N(0, 1). The KV pool has the reference's layout (kv_cache.py:20-50):
@@ -160,9 +161,20 @@ class DecodeStep:
               attend: Callable[[int, torch.Tensor], torch.Tensor]) -> torch.Tensor:  # fmt: skip
         """One decoder layer (model.py:137-179, the fused path): the new tokens' k/v go to
         the pool at ``slots``; ``attend(i, q)`` returns the attention output for ``q``."""
+        return x.add_(self._layer(i, x, None, cos, sin, slots, attend))
+
+    def _layer(self, i: int, x: torch.Tensor, pending: torch.Tensor | None, cos: torch.Tensor, sin: torch.Tensor,
+               slots: torch.Tensor, attend: Callable[[int, torch.Tensor], torch.Tensor]) -> torch.Tensor:  # fmt: skip
+        """``layer`` but for its last residual add, which it returns (for the next layer's
+        norm to make in the same pass); ``pending`` is the previous layer's. ``x`` is updated
+        in place: it is this step's own activation."""
         s, w, p = self.shape, self.w, f"model.layers.{i}."
         n = x.shape[0]
-        h = hip_fused.rms_norm_rows(x, w[p + "input_layernorm.weight"], s.rms_norm_eps)
+        norm = w[p + "input_layernorm.weight"]
+        if pending is None:
+            h = hip_fused.rms_norm_rows(x, norm, s.rms_norm_eps)
+        else:
+            h = hip_fused.add_rms_norm_rows(x, pending, norm, s.rms_norm_eps)
         qkv = F.linear(h, w[p + "self_attn.qkv_proj.weight"])
         q, k, v = torch.split(qkv, [s.q_size, s.kv_size, s.kv_size], dim=1)
         q = hip_fused.qk_norm_rope_store(
@@ -172,11 +184,11 @@ class DecodeStep:
             self.pool.v[i], s.rms_norm_eps)  # fmt: skip
         attn = attend(i, q)
         # Residual adds as model.py:172,179 writes them: the projection is rounded to the
-        # model dtype, then the sum (in place: x is this step's own activation).
-        x.add_(F.linear(attn.reshape(n, s.q_size), w[p + "self_attn.o_proj.weight"]))
-        h = hip_fused.rms_norm_rows(x, w[p + "post_attention_layernorm.weight"], s.rms_norm_eps)
-        gate, up = F.linear(h, w[p + "mlp.gate_up_proj.weight"]).chunk(2, dim=1)
-        return x.add_(F.linear(F.silu(gate) * up, w[p + "mlp.down_proj.weight"]))
+        # model dtype, then the sum.
+        h = hip_fused.add_rms_norm_rows(x, F.linear(attn.reshape(n, s.q_size), w[p + "self_attn.o_proj.weight"]),
+                                        w[p + "post_attention_layernorm.weight"], s.rms_norm_eps)  # fmt: skip
+        act = hip_fused.silu_mul(F.linear(h, w[p + "mlp.gate_up_proj.weight"]))
+        return F.linear(act, w[p + "mlp.down_proj.weight"])
 
     def _layers_rows(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slots: torch.Tensor,
                      attend: Callable[[int, torch.Tensor], torch.Tensor]) -> torch.Tensor:  # fmt: skip
@@ -214,9 +226,13 @@ class DecodeStep:
         if self.projections == "rows" and x.shape[0] <= ROWS_MAX:
             x = self._layers_rows(x, cos, sin, slots, attend)
         else:
+            pending = None
             for i in range(s.num_layers):
-                x = self.layer(i, x, cos, sin, slots, attend)
-            x = hip_fused.rms_norm_rows(x, self.w["model.norm.weight"], s.rms_norm_eps)
+                pending = self._layer(i, x, pending, cos, sin, slots, attend)
+            if pending is None:
+                x = hip_fused.rms_norm_rows(x, self.w["model.norm.weight"], s.rms_norm_eps)
+            else:
+                x = hip_fused.add_rms_norm_rows(x, pending, self.w["model.norm.weight"], s.rms_norm_eps)
         if rows is not None:
             x = x[rows]
         n = x.shape[0]
@@ -248,7 +264,10 @@ class DecodeStep:
 
         if one:
             d_idx = host_ints(one, torch.int64, dev)
-            d_rows = host_ints([starts[b] for b in one], torch.int64, dev)
+            # Decode rows side by side (prompts first, or last) are read and written in place.
+            d_lo, d_hi = starts[one[0]], starts[one[-1]] + 1
+            in_place = d_hi - d_lo == len(one)
+            d_rows = None if in_place else host_ints([starts[b] for b in one], torch.int64, dev)
             d_tables, d_lens = batch.block_tables[d_idx], batch.context_lens[d_idx]
         if rest:
             p_idx = host_ints(rest, torch.int64, dev)
@@ -262,7 +281,10 @@ class DecodeStep:
                 return hip_attention.launch_paged_decode_split(
                     q, k, v, batch.block_tables, batch.context_lens, scale, bs, self.num_splits)
             out = torch.empty_like(q)
-            if one:
+            if one and in_place:
+                hip_attention.launch_paged_decode_split_into(
+                    q[d_lo:d_hi], k, v, d_tables, d_lens, scale, bs, out[d_lo:d_hi], self.num_splits)  # fmt: skip
+            elif one:
                 out[d_rows] = hip_attention.launch_paged_decode_split(
                     q[d_rows], k, v, d_tables, d_lens, scale, bs, self.num_splits)  # fmt: skip
             hip_prefill.paged_prefill_attention(q, k, v, p_tables, p_starts, p_qlens, p_lens, scale, bs,

@@ -221,12 +221,14 @@ def _launch(
     block_size: int,
     splits: int,
     head_tile: int,
+    out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     dev = _lib.require_device(q, k_cache, v_cache, block_tables, context_lens)
     _check_kernel_shape(q, k_cache)
     b, hq, d = q.shape
     hkv = k_cache.shape[1]
-    out = torch.empty_like(q)
+    if out is None:
+        out = torch.empty_like(q)
     if b == 0:
         return out
     stream = _lib.stream_of(dev)
@@ -392,6 +394,27 @@ def launch_paged_decode_split(
     # No count given (None or 0): the policy.
     splits = num_splits or _policy_splits(q, k_cache, block_tables, block_size)
     return _launch(q, k_cache, v_cache, block_tables, context_lens, scale, block_size, splits, 0)
+
+
+def launch_paged_decode_split_into(
+    q: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    block_tables: torch.Tensor,
+    context_lens: torch.Tensor,
+    scale: float,
+    block_size: int,
+    out: torch.Tensor,
+    num_splits: int | None = None,
+) -> torch.Tensor:
+    """``launch_paged_decode_split`` into ``out`` (like q; rows of a larger tensor will do):
+    the one-token rows of a mixed step's flat batch, without gathering or scattering them."""
+    if num_splits and not 1 <= num_splits <= MAX_SPLITS:
+        raise ValueError(f"num_splits must be 1..{MAX_SPLITS}, got {num_splits}")
+    if out.shape != q.shape or out.dtype != q.dtype or out.stride(2) != 1 or out.device != q.device:
+        raise ValueError(f"out must be like q {tuple(q.shape)} {q.dtype}")
+    splits = num_splits or _policy_splits(q, k_cache, block_tables, block_size)
+    return _launch(q, k_cache, v_cache, block_tables, context_lens, scale, block_size, splits, 0, out)
 
 
 def launch_paged_decode_split_noalloc(

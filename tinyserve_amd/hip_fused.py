@@ -20,6 +20,7 @@ multiply by the weight in the input dtype, rotate in fp32 without fused multiply
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
 
 from tinyserve_amd import _lib
 
@@ -38,6 +39,47 @@ def rms_norm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Te
                   x.shape[0], x.shape[1], x.stride(0), out.stride(0), float(eps),
                   _lib.dtype_code(x), _lib.stream_of(dev))  # fmt: skip
     return out
+
+
+def add_rms_norm_rows(x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """``x.add_(y)`` then ``rms_norm_rows(x, weight, eps)``, in one launch where the rows fit
+    a wave's registers (up to 4096 16-bit elements, 16-byte aligned), else in two."""
+    if x.dim() != 2 or x.stride(1) != 1 or weight.shape != (x.shape[1],):
+        raise ValueError(f"need a row-contiguous [T, N] tensor and an [N] weight: {x.shape}")
+    if y.shape != x.shape or y.dtype != x.dtype or y.stride(1) != 1:
+        raise ValueError(f"y must be row-contiguous {tuple(x.shape)} {x.dtype}, got {tuple(y.shape)} {y.dtype}")
+    if weight.dtype != x.dtype or weight.stride(0) != 1:
+        raise ValueError(f"the weight must be a contiguous {x.dtype} vector, got {weight.dtype}")
+    out = torch.empty_like(x)
+    if x.shape[0]:
+        dev = _lib.require_device(x, y, weight)
+        rc = _lib.call_status("ts_add_rms_norm_rows", x.data_ptr(), y.data_ptr(), weight.data_ptr(), out.data_ptr(),
+                              x.shape[0], x.shape[1], x.stride(0), y.stride(0), out.stride(0), float(eps),
+                              _lib.dtype_code(x), _lib.stream_of(dev))  # fmt: skip
+        if rc == _lib.TS_EUNSUPPORTED:
+            return rms_norm_rows(x.add_(y), weight, eps)
+        if rc:
+            raise ValueError(f"ts_add_rms_norm_rows: {_lib.load().ts_strerror(rc).decode()}")
+    return out
+
+
+def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
+    """``F.silu(gate) * up`` of ``[gate | up]`` rows ``[T, 2N]``, as one launch where the rows
+    are 16-byte vectors, else by torch."""
+    if gate_up.dim() != 2 or gate_up.stride(1) != 1 or gate_up.shape[1] % 2:
+        raise ValueError(f"need row-contiguous [T, 2N] rows, got {tuple(gate_up.shape)}")
+    t, n = gate_up.shape[0], gate_up.shape[1] // 2
+    act = torch.empty(t, n, dtype=gate_up.dtype, device=gate_up.device)
+    if t and n:
+        dev = _lib.require_device(gate_up)
+        rc = _lib.call_status("ts_silu_mul", gate_up.data_ptr(), act.data_ptr(), t, n, gate_up.stride(0),
+                              act.stride(0), _lib.dtype_code(gate_up), _lib.stream_of(dev))  # fmt: skip
+        if rc == _lib.TS_EUNSUPPORTED:
+            gate, up = gate_up.chunk(2, dim=1)
+            return F.silu(gate) * up
+        if rc:
+            raise ValueError(f"ts_silu_mul: {_lib.load().ts_strerror(rc).decode()}")
+    return act
 
 
 def qk_norm_rope_store(
