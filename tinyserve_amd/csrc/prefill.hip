@@ -1040,20 +1040,30 @@ static int dispatch_hg_w(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows,
 }
 
 // Which of the three workgroup shapes a launch runs (see the header comment). wg8 is the
-// 8-wave grid. Measured at Qwen3 shapes: chunks of at most 128 new tokens (prefix hits)
-// run the 8-wave shape (+2.5-9.5%); grids under 1.5 8-wave workgroups per CU (one or two
-// long prompts) the 4-wave, 64-key shape at two per CU; grids of 1.5 to 8 per CU (3-16
-// prompts of 2048, 1-4 of 4096-8192: +1-10%), and of up to 16 per CU when the mean new
-// tokens per sequence is at most 1280 (8-32 mixed prompts, 16 x 512, 64 x 256: +5-14%),
-// the 4-wave, 32-key shape at three per CU; larger grids the 8-wave shape.
+// 8-wave grid, n4 the key-split shape's workgroups with query tiles in them (counted from
+// the rows where the host knows them: a grid sized by the longest of mixed prompts is mostly
+// empty), max_keys a bound on every context (0: unknown). The key-split shape runs one
+// workgroup per CU: it wins while one round holds them all, and in two rounds only on long
+// walks; the 4-wave, 32-key shape (three per CU) takes what is left of the small and
+// mid-size launches. Measured, us (16 q / 8 kv heads, D = 128, fp16, key-split / 32-key /
+// 8-wave): 1 x 64 7.3 / 5.7 / 5.6, 8 x 128 8.8 / 7.5 / 8.9, 1 x 512 12.7 / 14.2 / 16.7,
+// 4 x 512 14.7 / 15.9 / 18.2, 8 x 512 23.4 / 19.8 / 21.7, 16 x 200 19.0 / 14.1 / 14.0, six
+// prompts of 355-576 20.3 / 18.4 / 19.4, three of up to 2294 36.2 / 49.0 / 56.7, 2 x 2048
+// 45.8 / 51.8 / 55.8; 32 / 8 heads: 5 x 300 17.7 / 12.6 / 13.9, 3 x 700 30.4 / 23.3 / 24.2,
+// 1 x 1024 20.4 / 23.9 / 28.8. Grids of up to 8 8-wave workgroups per CU (3-16 prompts of
+// 2048, 1-4 of 4096-8192: +1-10%), and of up to 16 when the mean new tokens per sequence is
+// at most 1280 (8-32 mixed prompts: +5-14%), the 32-key shape; larger grids the 8-wave one.
 enum class PrefillShape { kW8, kW4, kW4Short };
 
-static PrefillShape prefill_shape(int R, int group, int Hkv, int max_q_len, int64_t n_rows) {
+static PrefillShape prefill_shape(int R, int group, int Hkv, int D, int max_q_len, int64_t n_rows,
+                                  int64_t max_keys) {
   const int hg8 = group < 8 ? group : 8;
   const int64_t wg8 = static_cast<int64_t>((max_q_len + 32 * (8 / hg8) - 1) / (32 * (8 / hg8))) *
                       R * Hkv * (group / hg8);
   const int64_t cus = compute_units();
   if (group > 4) return PrefillShape::kW8;
+  // Up to 128 new tokens and no long cached prefix: a few key tiles, all start and end.
+  if (max_q_len <= 128 && max_keys > 0 && max_keys <= 256) return PrefillShape::kW4Short;
   // Up to 64 new tokens per sequence in a launch of at most half an 8-wave workgroup per
   // CU: the key-split shape (its 64 queries hold each sequence, and it halves every walk
   // of the long cached prefix; +5-25% there, -4% to -11% in larger launches).
@@ -1061,7 +1071,13 @@ static PrefillShape prefill_shape(int R, int group, int Hkv, int max_q_len, int6
   // Up to 128 new tokens per sequence: one 8-wave query tile holds a whole sequence, so
   // its K/V (the whole cached prefix) is read once per kv head, not once per 64 queries.
   if (max_q_len <= 128) return PrefillShape::kW8;
-  if (2 * wg8 < 3 * cus) return PrefillShape::kW4;
+  const int oq = 32 * (4 / group);
+  const int64_t longest = static_cast<int64_t>(R) * ((max_q_len + oq - 1) / oq);
+  const bool mixed = n_rows > 0 && n_rows < static_cast<int64_t>(R) * max_q_len;
+  const int64_t n4 = Hkv * (mixed ? std::min(longest, n_rows / oq + (R + 1) / 2) : longest);
+  const int64_t mean = mixed ? n_rows / R : max_q_len;
+  const bool one_round = 100 * n4 <= (D == 64 ? 115 : 110) * cus;
+  if (one_round ? mean >= (D == 64 ? 100 : 224) : max_q_len * cus >= 1000 * n4) return PrefillShape::kW4;
   const bool short_mean = n_rows > 0 && n_rows <= 1280 * static_cast<int64_t>(R);
   if (wg8 <= 8 * cus || (short_mean && wg8 <= 16 * cus)) return PrefillShape::kW4Short;
   return PrefillShape::kW8;
@@ -1099,7 +1115,7 @@ static bool cut_shape(int R, int group, int Hkv, int D, int lbs, int max_q_len, 
   if (items > kWave) return false;
   // What a cut can gain, in steps of the longest workgroup of the shape that runs
   // otherwise (`fill`: its workgroups per CU).
-  const bool halves = prefill_shape(R, group, Hkv, max_q_len, 0) == PrefillShape::kW4;
+  const bool halves = prefill_shape(R, group, Hkv, D, max_q_len, 0, max_keys) == PrefillShape::kW4;
   if (!halves && max_q_len > 128) return false;
   const int hg = halves ? std::min(group, 4) : std::min(group, 8);
   const int oq = 32 * ((halves ? 4 : 8) / hg);
@@ -1154,8 +1170,9 @@ static int dispatch_cut(PrefillArgs& a, const CutShape& c, int Hkv, hipStream_t 
 }
 
 template <typename T, int D>
-static int dispatch_hg(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows, hipStream_t stream) {
-  switch (prefill_shape(a.R, a.group, Hkv, max_q_len, n_rows)) {
+static int dispatch_hg(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows, int64_t max_keys,
+                       hipStream_t stream) {
+  switch (prefill_shape(a.R, a.group, Hkv, D, max_q_len, n_rows, max_keys)) {
     case PrefillShape::kW4Short: return dispatch_hg_w<T, D, 4, 2, 32, 3>(a, Hkv, max_q_len, n_rows, stream);
     case PrefillShape::kW4:
       // Two key halves per workgroup (8 waves, one workgroup and two waves per SIMD per
@@ -1238,11 +1255,11 @@ extern "C" int ts_prefill_varlen_ws(const void* q, const void* k_cache, const vo
       return D == 64 ? dispatch_cut<bf16, 64>(a, c, Hkv, st) : dispatch_cut<bf16, 128>(a, c, Hkv, st);
     }
     if (dtype == TS_F16) {
-      return D == 64 ? dispatch_hg<f16, 64>(a, Hkv, max_q_len, n_rows, st)
-                     : dispatch_hg<f16, 128>(a, Hkv, max_q_len, n_rows, st);
+      return D == 64 ? dispatch_hg<f16, 64>(a, Hkv, max_q_len, n_rows, max_keys, st)
+                     : dispatch_hg<f16, 128>(a, Hkv, max_q_len, n_rows, max_keys, st);
     }
-    return D == 64 ? dispatch_hg<bf16, 64>(a, Hkv, max_q_len, n_rows, st)
-                   : dispatch_hg<bf16, 128>(a, Hkv, max_q_len, n_rows, st);
+    return D == 64 ? dispatch_hg<bf16, 64>(a, Hkv, max_q_len, n_rows, max_keys, st)
+                   : dispatch_hg<bf16, 128>(a, Hkv, max_q_len, n_rows, max_keys, st);
   }
   return prefill_rows_generic(q, k_cache, v_cache, out, block_tables, q_starts, q_lens,
                               context_lens, R, Hq, Hkv, D, lbs, max_q_len, q_stride_t,
