@@ -160,6 +160,27 @@ def test_policy_splits_for_small_grids(lib: ctypes.CDLL) -> None:
     assert policy(16, 128) == 1  # half the chip: one launch
 
 
+def test_compiled_binding_passes_the_declared_arguments(lib: ctypes.CDLL) -> None:
+    # fastcall.c against the ctypes signatures: every entry's kinds in order, and the same
+    # status for the same arguments.
+    from tinyserve_amd import _fastcall
+
+    kinds = {_lib._vp: "P", _lib._i: "I", _lib._i64: "L", _lib._f: "F", ctypes.c_double: "F"}
+    source = (Path(_lib.__file__).parent / "csrc" / "fastcall.c").read_text()
+    entries = re.findall(r"^ENTRY\((\w+), (\d+),\n(.*?)\)$", source, re.M | re.S)
+    assert {name for name, _, _ in entries} == set(_lib._fns) & {n for n in dir(_fastcall) if n.startswith("ts_")}
+    for name, count, args in entries:
+        want = [kinds[t] for t in _lib.SIGNATURES[name][1]]
+        got = re.findall(r"([PILF])\((\d+)\)", args)
+        assert [k for k, _ in got] == want and [int(i) for _, i in got] == list(range(int(count)))
+        with pytest.raises(TypeError):
+            getattr(_fastcall, name)(1)
+        zeros = [0.0 if k == "F" else None if k == "P" else 0 for k in want]
+        assert getattr(_fastcall, name)(*zeros) == getattr(lib, name)(*zeros)
+    with pytest.raises(TypeError):
+        _fastcall.ts_silu_mul("x", 0, 0, 0, 0, 0, 0, 0)
+
+
 def test_policy_runs_short_tables_as_one_launch(lib: ctypes.CDLL) -> None:
     # Small grids over short tables: 512 tokens x heads per wave, both sides of the line,
     # for one, two and four (of eight) heads a wave.

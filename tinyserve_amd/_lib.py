@@ -98,18 +98,41 @@ def load() -> ctypes.CDLL:
                 fn = getattr(lib, name)
                 fn.restype = res
                 fn.argtypes = args
+            _bind_fast(lib)
             _lib = lib
     return _lib
 
 
+# Entry points as ``call`` and ``call_status`` invoke them: through the compiled binding
+# where it has the name (fastcall.c), else through ctypes.
 _fns: dict[str, object] = {}
+
+
+def _bind_fast(lib: ctypes.CDLL) -> None:
+    """Fill ``_fns`` with the compiled binding's functions, pointed at ``lib``'s entry points
+    (none without the built module: every call then goes through ctypes)."""
+    try:
+        from tinyserve_amd import _fastcall
+    except ImportError:
+        return
+    for name in EXPORTS:
+        if _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value):
+            _fns[name] = getattr(_fastcall, name)
+
+
+def _fn(name: str) -> object:
+    lib = load()  # fills in the compiled binding's names
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(lib, name)
+    return fn
 
 
 def call(name: str, *args: object) -> None:
     """Call entry point ``name``; raise on a non-zero status."""
     fn = _fns.get(name)
     if fn is None:
-        fn = _fns[name] = getattr(load(), name)
+        fn = _fn(name)
     rc = fn(*args)
     if rc != 0:
         msg = load().ts_strerror(rc).decode()
@@ -123,7 +146,7 @@ def call_status(name: str, *args: object) -> int:
     positive status), so the caller can take another path on a TS_E* code."""
     fn = _fns.get(name)
     if fn is None:
-        fn = _fns[name] = getattr(load(), name)
+        fn = _fn(name)
     rc = fn(*args)
     if rc > 0:
         raise RuntimeError(f"{name}: HIP error {rc}: {load().ts_strerror(rc).decode()}")
@@ -145,16 +168,21 @@ def require_device(*tensors: torch.Tensor) -> int:
     fallback)."""
     idx = -1
     for t in tensors:
-        if not t.is_cuda:
+        i = t.get_device()
+        if i != idx:
+            if i < 0 or not t.is_cuda:
+                raise RuntimeError(
+                    "tinyserve_amd kernels run on a HIP device only (no CPU fallback); "
+                    f"got a tensor on {t.device}"
+                )
+            if idx >= 0:
+                raise ValueError(f"tensors on different devices: cuda:{idx} and cuda:{i}")
+            idx = i
+        elif i < 0:
             raise RuntimeError(
                 "tinyserve_amd kernels run on a HIP device only (no CPU fallback); "
                 f"got a tensor on {t.device}"
             )
-        i = t.get_device()
-        if idx < 0:
-            idx = i
-        elif i != idx:
-            raise ValueError(f"tensors on different devices: cuda:{idx} and cuda:{i}")
     return idx
 
 

@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -81,7 +82,23 @@ def build(verbose: bool = False) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     tmp.replace(out)  # atomic: a process that already mapped the old file keeps it
+    _build_fastcall(verbose)
     return out
+
+
+def _build_fastcall(verbose: bool) -> None:
+    """The compiled Python binding of the launch entry points (host code only)."""
+    cc = shutil.which("gcc") or shutil.which("cc") or hipcc()
+    out = PKG / "_fastcall.so"
+    tmp = out.with_suffix(".so.tmp")
+    cmd = [cc, "-O2", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}", str(CSRC / "fastcall.c"),
+           "-o", str(tmp)]  # fmt: skip
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"fastcall.c failed:\n{proc.stderr}")
+    tmp.replace(out)
 
 
 if __name__ == "__main__":

@@ -233,8 +233,7 @@ def _launch(
         return out
     stream = _lib.stream_of(dev)
     dt = _lib.dtype_code(q)
-    strides = (q.stride(0), q.stride(1), out.stride(0), out.stride(1),
-               k_cache.stride(0), k_cache.stride(1), block_tables.stride(0))  # fmt: skip
+    strides = (*q.stride()[:2], *out.stride()[:2], *k_cache.stride()[:2], block_tables.stride(0))
     width = block_tables.shape[1]  # bounds every context: picks the kernel's register budget
     if splits == 1:
         _lib.call("ts_decode_split", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),

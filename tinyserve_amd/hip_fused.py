@@ -146,8 +146,8 @@ def qk_norm_rope_store(
             q_weight.data_ptr(), k_weight.data_ptr(), cos.data_ptr(), sin.data_ptr(),
             slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
             t, num_q_heads, num_kv_heads, head_dim,
-            q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-            out.stride(0), out.stride(1), cos.stride(0), k_cache.stride(0), k_cache.stride(1),
+            *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], cos.stride(0),
+            *k_cache.stride()[:2],
             float(eps), _lib.dtype_code(q), _lib.dtype_code(k_cache), _lib.stream_of(dev),
         )  # fmt: skip
     return out

@@ -123,8 +123,7 @@ def paged_prefill_attention(
         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
         block_tables.data_ptr(), q_starts.data_ptr(), q_lens.data_ptr(), context_lens.data_ptr(),
         r, num_q_heads, num_kv_heads, head_dim, block_size, max_q_len, t,
-        q.stride(0), q.stride(1), out.stride(0), out.stride(1),
-        k_cache.stride(0), k_cache.stride(1), block_tables.stride(0),
+        *q.stride()[:2], *out.stride()[:2], *k_cache.stride()[:2], block_tables.stride(0),
         float(scale), _lib.dtype_code(q), max_keys, _lib.ptr(ws), floats, _lib.stream_of(dev),
     )  # fmt: skip
     return out
