@@ -207,3 +207,14 @@ def test_silu_mul_equals_torch(t: int, n: int, dtype: torch.dtype) -> None:
     ulp = {torch.float32: 2.0**-22, torch.float16: 2.0**-10, torch.bfloat16: 2.0**-7}[dtype]
     tiny = {torch.float32: 1e-30, torch.float16: 2.0**-23, torch.bfloat16: 1e-30}[dtype]
     assert ((got.double() - want.double()).abs() <= 2 * ulp * want.double().abs() + tiny * (1 + up.abs())).all()
+
+
+@pytest.mark.parametrize("t", [2047, 2049, 8191, 8195])
+def test_rope_tables_of_many_positions(t: int) -> None:
+    # Two and four positions per thread (from 2048 and 8192 at D = 128), whole and cut last
+    # threads: every row equals the row of a short launch.
+    pos = torch.randint(0, 40960, (t,), generator=torch.Generator().manual_seed(t)).to(DEVICE)
+    cos, sin = rope_cos_sin(128, 1.0e6, pos)
+    for at in (0, t // 2, t - 5):
+        c, s = rope_cos_sin(128, 1.0e6, pos[at : at + 5])
+        assert torch.equal(cos[at : at + 5], c) and torch.equal(sin[at : at + 5], s)

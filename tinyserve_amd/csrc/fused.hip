@@ -396,23 +396,34 @@ static int launch_qk_cache(const QkArgs& a, int D, int cache_dtype, hipStream_t 
 }
 
 // ---------------------------------------------------------------------------------
-// rope_cos_sin: the rotation tables of layers.py:41-65 for T positions, one thread per
-// (position, pair i): inv_freq = theta^(-2i / D) and the angle p * inv_freq in float64,
-// cos / sin in float64 rounded once to float32, written to columns i and i + D/2.
+// rope_cos_sin: the rotation tables of layers.py:41-65 for T positions: inv_freq = theta^(-2i
+// / D) and the angle p * inv_freq in float64, cos / sin in float64 rounded once to float32,
+// written to columns i and i + D/2. Bound by the float64 functions: a thread takes PPT
+// positions of one pair i, so the power is computed once for them. Measured at D = 128, one /
+// two / four positions a thread: 4096 positions 5.1 / 4.5 / 4.7 us, 16384 14.3 / 11.4 / 10.1.
+template <int PPT>
 __global__ __launch_bounds__(256) void rope_cos_sin_kernel(const int64_t* __restrict__ pos, int T, int D,
                                                            double theta, float* __restrict__ cos_out,
                                                            float* __restrict__ sin_out, int64_t stride) {
   const int half = D / 2;
   const int64_t u = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (u >= static_cast<int64_t>(T) * half) return;
-  const int t = static_cast<int>(u / half), i = static_cast<int>(u % half);
+  const int t0 = static_cast<int>(u / half) * PPT, i = static_cast<int>(u % half);
+  if (t0 >= T) return;
+  int64_t p[PPT];
+#pragma unroll
+  for (int k = 0; k < PPT; ++k) p[k] = t0 + k < T ? pos[t0 + k] : 0;
   const double inv_freq = pow(theta, -static_cast<double>(2 * i) / static_cast<double>(D));
-  const double ang = static_cast<double>(pos[t]) * inv_freq;
-  const float c = static_cast<float>(cos(ang)), sn = static_cast<float>(sin(ang));
-  cos_out[t * stride + i] = c;
-  cos_out[t * stride + i + half] = c;
-  sin_out[t * stride + i] = sn;
-  sin_out[t * stride + i + half] = sn;
+#pragma unroll
+  for (int k = 0; k < PPT; ++k) {
+    const int64_t t = t0 + k;
+    if (t >= T) break;
+    const double ang = static_cast<double>(p[k]) * inv_freq;
+    const float c = static_cast<float>(cos(ang)), sn = static_cast<float>(sin(ang));
+    cos_out[t * stride + i] = c;
+    cos_out[t * stride + i + half] = c;
+    sin_out[t * stride + i] = sn;
+    sin_out[t * stride + i + half] = sn;
+  }
 }
 
 }  // namespace ts
@@ -424,9 +435,22 @@ extern "C" int ts_rope_cos_sin(const int64_t* positions, int T, int D, double th
   if (T < 0 || D < 2 || D % 2 || stride < D || !(theta > 0.0)) return TS_EINVAL;
   if (T == 0) return 0;
   if (!positions || !cos_out || !sin_out) return TS_EINVAL;
+  hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t n = static_cast<int64_t>(T) * (D / 2);
-  hipLaunchKernelGGL(rope_cos_sin_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), positions, T, D, theta, cos_out, sin_out, stride);
+  // Two positions per thread from one wave per SIMD of such threads on, four from two.
+  const int64_t lanes = 4 * 64 * static_cast<int64_t>(compute_units());
+  if (n >= 8 * lanes) {
+    const int64_t n4 = static_cast<int64_t>((T + 3) / 4) * (D / 2);
+    hipLaunchKernelGGL(rope_cos_sin_kernel<4>, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,
+                       positions, T, D, theta, cos_out, sin_out, stride);
+  } else if (n >= 2 * lanes) {
+    const int64_t n2 = static_cast<int64_t>((T + 1) / 2) * (D / 2);
+    hipLaunchKernelGGL(rope_cos_sin_kernel<2>, dim3(static_cast<unsigned>((n2 + 255) / 256)), dim3(256), 0, st,
+                       positions, T, D, theta, cos_out, sin_out, stride);
+  } else {
+    hipLaunchKernelGGL(rope_cos_sin_kernel<1>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st,
+                       positions, T, D, theta, cos_out, sin_out, stride);
+  }
   return launch_status();
 }
 
