@@ -610,3 +610,16 @@ def test_small_grid_policy_replays_in_a_graph(lens: list[int]) -> None:
         torch.cuda.synchronize()
         torch.testing.assert_close(got, want, atol=0, rtol=0)
         torch.randn(1 << 20, device=DEVICE).sum()  # unrelated eager work between replays
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,splits", [(40, 1), (40, 4), (40, 12), (16, None), (16, 1), (3, None), (70, 1)])
+def test_four_head_tiles_of_128_elements(batch: int, splits: int | None, dtype: torch.dtype) -> None:
+    # Two waves per SIMD: length pairs of eight waves (40), the in-group split ranges of eight
+    # waves and, where their states do not fit the LDS, of four (4 and 12 splits), plain
+    # workgroups of eight, the policy's partials, and several workgroups per CU (70).
+    c = decode_case([1 + (389 * i) % 1100 for i in range(batch)], 32, 8, dtype=dtype, seed=batch)
+    g = on_gpu(c)
+    out = ha.launch_paged_decode_split(*g.args(), c.scale, c.block_size, num_splits=splits)
+    assert_matches(out, oracle32(c), dtype, f"{batch} sequences, {splits} splits")

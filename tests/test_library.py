@@ -181,6 +181,15 @@ def test_compiled_binding_passes_the_declared_arguments(lib: ctypes.CDLL) -> Non
         _fastcall.ts_silu_mul("x", 0, 0, 0, 0, 0, 0, 0)
 
 
+def test_policy_splits_of_four_head_tiles(lib: ctypes.CDLL) -> None:
+    # Half the chip's SIMDs exactly (16 sequences of 8 eight-wave workgroups) is split into
+    # partials at four heads of 128 elements; more is one launch, as at two heads or 64.
+    policy = hip_attention.policy_splits
+    assert policy(16, 32, 8, 128, 16, 256) > 1
+    assert policy(17, 32, 8, 128, 16, 256) == 1 and policy(48, 32, 8, 128, 16, 256) == 1
+    assert policy(16, 16, 8, 128, 16, 256) == 1
+
+
 def test_policy_runs_short_tables_as_one_launch(lib: ctypes.CDLL) -> None:
     # Small grids over short tables: 512 tokens x heads per wave, both sides of the line,
     # for one, two and four (of eight) heads a wave.

@@ -48,9 +48,15 @@ namespace ts {
 // waves all run in one round, where each wave must keep much in flight. kLight: 32 bytes
 // per lane, two in flight, two waves per SIMD -- for launches of several rounds, where
 // the second wave per SIMD hides each wave's start-up chain (lengths, block table, first
-// loads) and merge. (Tiles of four query heads stream 16 bytes per lane under it, or
-// their state would spill.) kLightStream is kLight with K/V read by non-temporal loads,
+// loads) and merge. (Tiles of four query heads of under 128 elements stream 16 bytes per lane
+// under it: short walks merge less, 8 x 128 at D = 64 6.6 us against 7.4 at 32.) Decode tiles
+// of four heads of 128 elements or more run the light registers under either budget: at 64
+// bytes per lane an iteration was ~3000 cycles of one wave's chain, which a
+// second wave per SIMD hides (32 q / 8 kv heads bf16, us: 16 x 1024 32.7 -> 26.1, 16 x 4096
+// 85 -> 77, 48 x U[100, 5000] 116 -> 108, 64 x U[1, 2048] 58 -> 53, 128 x 4096 384 -> 371).
+// kLightStream is kLight with K/V read by non-temporal loads,
 // for decode launches larger than the last-level cache.
+constexpr bool two_per_simd(int ht, int d) { return ht == 4 && d >= 128; }
 enum Budget { kHeavy = 0, kLight = 1, kLightStream = 2 };
 template <int B>
 struct BudgetOf {
@@ -350,8 +356,7 @@ template <typename T, int D, int HT, bool PREFILL, int BUDGET, bool CUT = false>
 __global__ __launch_bounds__(PREFILL ? kWave : kWave * (BudgetOf<BUDGET>::kLightish ? kMaxWavesLight : kMaxWavesPerGroup))
 __attribute__((amdgpu_waves_per_eu(BudgetOf<BUDGET>::kWavesPerEU)))
 void paged_attend_kernel(const AttendArgs a) {
-  // Under the light budget four query heads' state fits only at 16 bytes per lane.
-  constexpr int LB = BudgetOf<BUDGET>::kLightish && HT == 4 ? 16 : BudgetOf<BUDGET>::kLaneBytes;
+  constexpr int LB = BudgetOf<BUDGET>::kLightish && HT == 4 && D < 128 ? 16 : BudgetOf<BUDGET>::kLaneBytes;
   using S = RowShape<T, D, LB>;
   constexpr int LPT = S::kLPT, NV = S::kNV, VEC = S::kVec, TPW = S::kTPW, E = S::kE;
   // Streaming launches are bound by issue, cached ones (short walks) by latency.
@@ -865,38 +870,39 @@ static int launch_attend(const AttendArgs& a, dim3 grid, bool light, size_t lds,
   if constexpr (!PREFILL) {
     if (a.cuts > 1) {
       // In-workgroup split-K over the reference's split ranges (cut mode).
-      if constexpr (D == 64 || D == 128) {
+      if constexpr (HT < 4 && (D == 64 || D == 128)) {
         if (light && a.stream_kv) {
           hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kLightStream, true>), grid,
                              dim3(kWave * a.wpg), lds, stream, a);
           return launch_status();
         }
       }
-      if (light)
+      if (light || two_per_simd(HT, D))
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kLight, true>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
-      else
+      else if constexpr (!two_per_simd(HT, D))
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kHeavy, true>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
       return launch_status();
     }
   }
   {
-    if constexpr (!PREFILL && (D == 64 || D == 128)) {
+    if constexpr (!PREFILL && HT < 4 && (D == 64 || D == 128)) {
       if (light && a.stream_kv) {
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kLightStream>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
         return launch_status();
       }
     }
-    if (light) {
+    if (light || (!PREFILL && two_per_simd(HT, D))) {
       hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kLight>), grid,
                          dim3(kWave * a.wpg), lds, stream, a);
       return launch_status();
     }
   }
-  hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kHeavy>), grid, dim3(kWave * a.wpg),
-                     lds, stream, a);
+  if constexpr (PREFILL || !two_per_simd(HT, D))
+    hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kHeavy>), grid, dim3(kWave * a.wpg),
+                       lds, stream, a);
   return launch_status();
 }
 
@@ -1000,7 +1006,7 @@ struct DecodePlan {
 
 // Tokens one wave streams per loop iteration (TPW of the kernel's RowShape).
 static int tokens_per_iteration(int dtype, int D, int ht, int budget) {
-  const int lb = budget != kHeavy ? (ht == 4 ? 16 : 32) : 64;
+  const int lb = two_per_simd(ht, D) ? 32 : budget != kHeavy ? (ht == 4 ? 16 : 32) : 64;
   const int row = D * (dtype == TS_F32 ? 4 : 2);
   const int lpt = row <= lb ? 1 : std::min(row / lb, kWave);
   return kWave / lpt;
@@ -1047,17 +1053,15 @@ static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_bl
   const int64_t kv_bytes = static_cast<int64_t>(B) * max_blocks * block_size * Hkv * D *
                            (dtype == TS_F32 ? 4 : 2) * 2;
   const bool stream_kv = max_blocks > 0 && (D == 64 || D == 128) && kv_bytes > (int64_t{256} << 20);
-  // Tiles of four query heads stream 16 bytes per lane under the light budget; they run
-  // the heavy budget instead (64 bytes per lane, three iterations in flight, one wave per
-  // SIMD) with cached loads, which also let the second tile of a kv head's blocks (groups
-  // of eight) read them from L2. Measured against the light streaming launch: 64 x 4096
-  // with 32 / 8 heads 207 -> 193 us, 128 x 4096 407 -> 379 us, 64 / 8 heads 406 -> 328
-  // us, 16 x 8192 bf16 208 -> 158 us; with non-temporal loads the heavy launch took
-  // 212, 424, 426 and 186 us. Rows of 64 elements likewise (64 x 4096 130 -> 120 us,
-  // 64 x 8192 257 -> 233 us); two-head tiles of 128-element rows keep the light budget
-  // (the heavy one: 184 against 160 us at 64 x 4096).
+  // Tiles of four query heads keep cached loads (the heavy budget's), which also let the
+  // second tile of a kv head's blocks (groups of eight) read them from L2. Measured at 32 /
+  // 8 heads bf16, cached against non-temporal: 64 x U[1, 2048] 52.7 against 58.8 us, 16 x
+  // U[100, 5000] 91 against 97, but 64 x 4096 193 against 188. Rows of 64 elements run the
+  // heavy budget (64 x 4096 130 -> 120 us, 64 x 8192 257 -> 233 us); two-head tiles of
+  // 128-element rows keep the light budget (the heavy one: 184 against 160 us at 64 x 4096).
   const bool heavy_stream = stream_kv && (ht == 4 || D == 64);
-  if (stream_kv && by_length) wpg = heavy_stream ? kMaxWavesPerGroup : kMaxWavesLight;
+  const bool two = two_per_simd(ht, D);
+  if (by_length && (two || (stream_kv && !heavy_stream))) wpg = kMaxWavesLight;
   // Cached launches of two-head tiles of 16-bit 128- or 64-element rows: the light budget
   // at any walk length (measured against heavy: equal or faster on every shape from
   // 32 x 256 to 64 x 1024 and 24 x 2048, e.g. 64 x 1024 45.2 -> 42.1 us; D=64 64 x 1024
@@ -1070,7 +1074,7 @@ static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_bl
   // that each walks fewer tokens (fewer dependent rounds of loads per wave).
   if (stream_kv && !by_length && !heavy_stream) {
     while (wpg < kMaxWavesLight && waves * wpg < 2 * want) wpg *= 2;
-  } else if (light && !by_length) {
+  } else if ((light || two) && !by_length) {
     while (wpg < kMaxWavesLight && waves * wpg * 2 <= 2 * want) wpg *= 2;
   }
   plan->ht = ht;
@@ -1133,7 +1137,11 @@ extern "C" int ts_decode_split(const void* q, const void* k_cache, const void* v
     // A piece ends at a split boundary between two loop iterations only if an
     // iteration's tokens never straddle a block; every piece's state needs an LDS slot.
     if (block_size % tokens_per_iteration(dtype, D, p.ht, p.budget)) return TS_EUNSUPPORTED;
-    lds = static_cast<size_t>((p.by_length ? 2 : 1) * (splits + p.wpg) * state_slot_bytes(p.ht, D));
+    // (A workgroup of eight waves drops to four to fit.)
+    const int per = (p.by_length ? 2 : 1) * static_cast<int>(state_slot_bytes(p.ht, D));
+    if (two_per_simd(p.ht, D) && p.wpg > kMaxWavesPerGroup && static_cast<size_t>(per) * (splits + p.wpg) > kMaxInGroupLds)
+      a.wpg = p.wpg = kMaxWavesPerGroup;
+    lds = static_cast<size_t>(per) * (splits + p.wpg);
     if (lds > kMaxInGroupLds) return TS_EUNSUPPORTED;
     a.cuts = splits;
   }

@@ -172,11 +172,12 @@ def decode_plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, 
 def _one_split_waves(device: int, b: int, hq: int, hkv: int, d: int, block_size: int, width: int,
                      dtype: torch.dtype) -> int:  # fmt: skip
     """SIMDs the one-split launch of these sizes occupies on ``device`` (which sets the CU
-    count): its waves, over the two waves per SIMD of the light budgets."""
+    count): its waves, over the two waves per SIMD of the light budgets and of four-head
+    tiles of 128 or more elements."""
     p = decode_plan(b, hq, hkv, d, block_size, width, 1, 0, dtype)
     gx, gy, gz = p["grid"]
     waves = gx * gy * gz * int(p["waves_per_group"])
-    return waves // 2 if p["budget"] in ("light", "light_stream") else waves
+    return waves // 2 if p["budget"] in ("light", "light_stream") or (p["head_tile"] == 4 and d >= 128) else waves
 
 
 def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int,
@@ -195,7 +196,9 @@ def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int
     heads = min(num_q_heads // num_kv_heads, 4)  # per wave
     if head_dim <= 128 and max_blocks * block_size * heads <= ONE_LAUNCH_TOKEN_HEADS:
         return 1
-    if simds >= IN_GROUP_MIN_WAVES // 2:
+    # Four-head tiles of 128 elements: just half the chip is not enough (32 q / 8 kv heads bf16
+    # 16 x 4096: one launch 78 us, partials 50; 16 x U[100, 5000] 91 and 56).
+    if simds >= IN_GROUP_MIN_WAVES // 2 + (heads == 4 and head_dim >= 128):
         return 1 if splits <= IN_GROUP_SPLITS else splits
     return max(splits, min(-(-2 * IN_GROUP_MIN_WAVES // max(simds, 1)), MAX_SPLITS, max_blocks))
 
