@@ -385,7 +385,16 @@ prefill_mfma_kernel(const PrefillArgs a) {
       if (__all(mine < (1 << 25))) {
         // Unique keys (length, then lower index first): rank = keys above this one.
         const int key = ln < a.R ? mine * kWave + (kWave - 1 - ln) : -1;
-        for (int j = 0; j < a.R; ++j) rank += __builtin_amdgcn_readlane(key, j) > key;
+        // Eight lanes at a time, their numbers immediate (lanes past R rank below all): a
+        // loop of one is mostly its own counting, paid by every workgroup.
+        // (us, fp16 at 16 / 8 heads: 64 prompts of U[16, 300] 35.5 -> 31.8, 32 of U[16, 2048]
+        // 188 -> 185.)
+#pragma unroll
+        for (int j0 = 0; j0 < kWave; j0 += 8) {
+          if (j0 >= a.R) break;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) rank += __builtin_amdgcn_readlane(key, j0 + j) > key;
+        }
       } else {
         for (int j = 0; j < a.R; ++j) {
           const int other = __builtin_amdgcn_readlane(mine, j);
