@@ -408,7 +408,14 @@ void paged_attend_kernel(const AttendArgs a) {
         if (__all(mine < (1 << 25))) {
           // Unique keys (length, then lower index first): rank = keys above this one.
           const int key = lane < B ? mine * kWave + (kWave - 1 - lane) : -1;
-          for (int j = 0; j < B; ++j) rank += __builtin_amdgcn_readlane(key, j) > key;
+          // Eight lanes at a time, their numbers immediate (lanes past B rank below all): 64 x
+          // U[1, 300] 15.6 -> 14.1 us, 64 x U[1024, 4096] 104 -> 103.
+#pragma unroll
+          for (int j0 = 0; j0 < kWave; j0 += 8) {
+            if (j0 >= B) break;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) rank += __builtin_amdgcn_readlane(key, j0 + j) > key;
+          }
         } else {
           for (int j = 0; j < B; ++j) {
             const int other = __builtin_amdgcn_readlane(mine, j);
