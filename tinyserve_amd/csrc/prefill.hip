@@ -39,7 +39,7 @@
 // w + 4 walk the lower and upper half of the key tiles (a 2-stage ring holding one tile
 // of each half, 128 KB) and merge their softmax states through LDS at the end, which
 // halves the longest workgroup's walk and puts two waves on each SIMD; and for mid-size
-// launches, 4 waves over 32-key tiles (a 2-stage ring of 34 KB, 157 VGPRs: three
+// launches and short prompts, 4 waves over 32-key tiles (a 2-stage ring of 34 KB, 157 VGPRs: three
 // workgroups, so three waves, per SIMD), whose extra wave per SIMD and finer key tiles
 // outweigh the doubled barriers there. (Block sizes under 4 slots, 8 at D=64, run 4
 // waves without the split: the halves' block ids come from the scalar-id gather.)

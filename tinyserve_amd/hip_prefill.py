@@ -9,7 +9,9 @@ workgroup. The library compiles three workgroup shapes and picks one from the la
 sizes: 8 waves over 64-key tiles (128 queries x 2 heads, a 3-stage ring; large launches),
 8 waves over 64 queries x 2 heads with the keys split into two halves walked by waves
 w and w + 4 and merged through LDS (launches too small to fill the chip), and 4 waves
-over 32-key tiles, three workgroups per CU (mid-size launches). fp16 P is rounded to
+over 32-key tiles, three workgroups per CU (mid-size launches and short prompts). Chunks
+behind long cached prefixes are cut along their keys over several workgroups, whose fp32
+states go through a workspace from torch's allocator and a second kernel. fp16 P is rounded to
 fp16 before P.V, as the reference kernel rounds P to V's dtype (triton_prefill.py:118);
 bf16 P is carried as a hi + lo bf16 pair (two P.V MFMAs), since one bf16 rounding moves
 outputs past the tolerance. fp32 inputs (exact fp32 dots, the reference's "ieee" path)
