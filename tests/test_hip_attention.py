@@ -433,11 +433,12 @@ def test_paired_sequences_of_2_to_the_25_tokens() -> None:
 @pytest.mark.parametrize("heads", [(16, 8), (32, 8)])
 def test_both_register_budgets(batch: int, splits: int, heads: tuple[int, int], dtype: torch.dtype) -> None:
     # The table width bounds the tokens a wave walks; under 512 of them the kernel runs
-    # its light budget (two waves per SIMD, up to 8 a workgroup; 16 bytes a lane for tiles
-    # of four query heads), else the heavy one. The same sequences through their own
-    # narrow table and through one widened to 2000 blocks give the reference either way:
-    # length pairs (64, 45), in-workgroup splits (32 x 4), a small batch, and HBM splits
-    # with the combine (8 x 8), at GQA groups of 2 and 4.
+    # its light budget (two waves per SIMD, up to 8 a workgroup), else, for fp32 at two
+    # heads a wave, the heavy one. (16-bit two-head tiles and four-head tiles of 128
+    # elements are light at any walk.) The same sequences through their own narrow table
+    # and through one widened to 2000 blocks give the reference either way: length pairs
+    # (64, 45), in-workgroup splits (32 x 4), a small batch, and HBM splits with the combine
+    # (8 x 8), at GQA groups of 2 and 4.
     lens = [1 + (389 * i) % 300 for i in range(batch)]
     c = decode_case(lens, num_q_heads=heads[0], num_kv_heads=heads[1], dtype=dtype, seed=batch)
     want = oracle32(c)
@@ -505,8 +506,8 @@ def test_combine_over_many_splits(splits: int, head_dim: int, dtype: torch.dtype
 def test_streaming_launches(dtype: torch.dtype, head_dim: int, heads: tuple[int, int], head_tile: int) -> None:
     # A table wide enough to bound more than 256 MiB of K/V makes the launch stream K/V
     # with non-temporal loads (light budget, one round of workgroups; tiles of four query
-    # heads and 64-element rows take the heavy budget's cached loads instead); the unused columns
-    # are never read. Head groups of 2, 4 and 1 (tiles of 2, 4 and 1 query heads) and the
+    # heads and 64-element rows keep cached loads, the latter under the heavy budget); the
+    # unused columns are never read. Head groups of 2, 4 and 1 (tiles of 2, 4 and 1 query heads) and the
     # per-head launch; 32 sequences give length pairs at one split. The results match the
     # oracle and the launch over the tight table, for one split and for HBM splits.
     lens = [1, 17, 300, 64, 1000, 5, 700, 33] * 4
@@ -518,10 +519,10 @@ def test_streaming_launches(dtype: torch.dtype, head_dim: int, heads: tuple[int,
     wide[:, :w] = g.block_tables
     for splits in (1, 4):
         plan = ha.decode_plan(b, *heads, head_dim, g.block_size, 8192, splits, head_tile, dtype)
-        # Tiles of four query heads and rows of 64 elements run the heavy budget with cached
-        # loads; the others stream.
-        heavy = plan["head_tile"] == 4 or head_dim == 64
-        assert plan["budget"] == ("heavy" if heavy else "light_stream"), plan
+        # Rows of 64 elements run the heavy budget and tiles of four query heads of 128 the
+        # light one, both with cached loads; the others stream.
+        cached = "heavy" if head_dim == 64 else "light" if plan["head_tile"] == 4 else None
+        assert plan["budget"] == (cached or "light_stream"), plan
         tight = ha._launch(*g.args(), g.scale, g.block_size, splits, head_tile)
         out = ha._launch(g.q, g.k_cache, g.v_cache, wide, g.context_lens, g.scale, g.block_size, splits,
                          head_tile)  # fmt: skip

@@ -130,18 +130,19 @@ def test_decode_launch_plans(lib: ctypes.CDLL) -> None:
 def test_decode_budget_choices(lib: ctypes.CDLL) -> None:
     # Which register budget a launch runs (sizes only). Streaming launches (K/V bounded by
     # the table width above 256 MiB): light-stream for two-head tiles of 128-element rows,
-    # the heavy budget's cached loads for four-head tiles and 64-element rows. Cached
-    # launches of two-head 16-bit tiles: light at any walk length; fp32 and four-head
-    # tiles keep the walk rule (heavy for long walks on one round of waves).
+    # cached loads under the heavy budget for 64-element rows. Four-head tiles of 128
+    # elements: light, cached, always. Cached launches of two-head 16-bit tiles: light at any
+    # walk length; fp32 keeps the walk rule (heavy for long walks on one round of waves).
     plan = hip_attention.decode_plan
     assert plan(64, 16, 8, 128, 16, 256, 1)["budget"] == "light_stream"
-    assert plan(64, 32, 8, 128, 16, 256, 1)["budget"] == "heavy"  # four-head tiles
+    assert plan(64, 32, 8, 128, 16, 256, 1)["budget"] == "light"  # four-head tiles
     assert plan(64, 32, 8, 128, 16, 256, 1)["head_tile"] == 4
     assert plan(64, 16, 8, 64, 16, 512, 1)["budget"] == "heavy"  # D=64, 512 MiB bound
     assert plan(64, 16, 8, 128, 16, 64, 1)["budget"] == "light"  # 64 x 1024, cached
     assert plan(16, 16, 8, 128, 16, 128, 1, dtype=torch.bfloat16)["budget"] == "light"
     assert plan(64, 16, 8, 64, 16, 64, 1)["budget"] == "light"  # D=64, cached
-    assert plan(64, 32, 8, 128, 16, 64, 1)["budget"] == "heavy"  # four heads, long walks
+    assert plan(64, 32, 8, 128, 16, 64, 1)["budget"] == "light"  # four heads, long walks
+    assert plan(64, 32, 8, 64, 16, 64, 1, dtype=torch.float32)["budget"] == "heavy"  # four of 64
     assert plan(8, 16, 8, 128, 16, 256, 1, dtype=torch.float32)["budget"] == "heavy"
 
 

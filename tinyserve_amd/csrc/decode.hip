@@ -50,7 +50,7 @@ namespace ts {
 // the second wave per SIMD hides each wave's start-up chain (lengths, block table, first
 // loads) and merge. (Tiles of four query heads of under 128 elements stream 16 bytes per lane
 // under it: short walks merge less, 8 x 128 at D = 64 6.6 us against 7.4 at 32.) Decode tiles
-// of four heads of 128 elements or more run the light registers under either budget: at 64
+// of four heads of 128 elements or more always run the light budget: at 64
 // bytes per lane an iteration was ~3000 cycles of one wave's chain, which a
 // second wave per SIMD hides (32 q / 8 kv heads bf16, us: 16 x 1024 32.7 -> 26.1, 16 x 4096
 // 85 -> 77, 48 x U[100, 5000] 116 -> 108, 64 x U[1, 2048] 58 -> 53, 128 x 4096 384 -> 371).
@@ -199,7 +199,7 @@ __device__ __forceinline__ void merge_token_lanes(TokenState<T, D, HT, LB>& st) 
   }
 }
 
-constexpr int kMaxWavesPerGroup = 4;  // heavy budget, and length pairs
+constexpr int kMaxWavesPerGroup = 4;  // heavy budget, and length pairs of cached launches
 constexpr int kMaxWavesLight = 8;     // light budget (two waves per SIMD)
 
 // LDS of a decode workgroup (dynamic, sized by the launch): NS state slots, each the
@@ -884,13 +884,17 @@ static int launch_attend(const AttendArgs& a, dim3 grid, bool light, size_t lds,
           return launch_status();
         }
       }
-      if (light || two_per_simd(HT, D))
+      if (light) {
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kLight, true>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
-      else if constexpr (!two_per_simd(HT, D))
+        return launch_status();
+      }
+      if constexpr (!two_per_simd(HT, D)) {
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kHeavy, true>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
-      return launch_status();
+        return launch_status();
+      }
+      return TS_EUNSUPPORTED;  // the plan gives these tiles the light budget
     }
   }
   {
@@ -901,16 +905,18 @@ static int launch_attend(const AttendArgs& a, dim3 grid, bool light, size_t lds,
         return launch_status();
       }
     }
-    if (light || (!PREFILL && two_per_simd(HT, D))) {
+    if (light) {
       hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kLight>), grid,
                          dim3(kWave * a.wpg), lds, stream, a);
       return launch_status();
     }
   }
-  if constexpr (PREFILL || !two_per_simd(HT, D))
+  if constexpr (PREFILL || !two_per_simd(HT, D)) {
     hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kHeavy>), grid, dim3(kWave * a.wpg),
                        lds, stream, a);
-  return launch_status();
+    return launch_status();
+  }
+  return TS_EUNSUPPORTED;  // the plan gives these tiles the light budget
 }
 
 template <typename T, bool PREFILL>
@@ -1013,7 +1019,7 @@ struct DecodePlan {
 
 // Tokens one wave streams per loop iteration (TPW of the kernel's RowShape).
 static int tokens_per_iteration(int dtype, int D, int ht, int budget) {
-  const int lb = two_per_simd(ht, D) ? 32 : budget != kHeavy ? (ht == 4 ? 16 : 32) : 64;
+  const int lb = budget == kHeavy ? 64 : ht == 4 && D < 128 ? 16 : 32;
   const int row = D * (dtype == TS_F32 ? 4 : 2);
   const int lpt = row <= lb ? 1 : std::min(row / lb, kWave);
   return kWave / lpt;
@@ -1060,34 +1066,34 @@ static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_bl
   const int64_t kv_bytes = static_cast<int64_t>(B) * max_blocks * block_size * Hkv * D *
                            (dtype == TS_F32 ? 4 : 2) * 2;
   const bool stream_kv = max_blocks > 0 && (D == 64 || D == 128) && kv_bytes > (int64_t{256} << 20);
-  // Tiles of four query heads keep cached loads (the heavy budget's), which also let the
-  // second tile of a kv head's blocks (groups of eight) read them from L2. Measured at 32 /
-  // 8 heads bf16, cached against non-temporal: 64 x U[1, 2048] 52.7 against 58.8 us, 16 x
-  // U[100, 5000] 91 against 97, but 64 x 4096 193 against 188. Rows of 64 elements run the
-  // heavy budget (64 x 4096 130 -> 120 us, 64 x 8192 257 -> 233 us); two-head tiles of
-  // 128-element rows keep the light budget (the heavy one: 184 against 160 us at 64 x 4096).
-  const bool heavy_stream = stream_kv && (ht == 4 || D == 64);
+  // Tiles of four query heads keep cached loads, which also let the second tile of a kv
+  // head's blocks (groups of eight) read them from L2. Measured at 32 / 8 heads bf16,
+  // cached against non-temporal: 64 x U[1, 2048] 52.7 against 58.8 us, 16 x U[100, 5000] 91
+  // against 97, but 64 x 4096 193 against 188. So do rows of 64 elements, under the heavy
+  // budget (64 x 4096 130 -> 120 us, 64 x 8192 257 -> 233 us); two-head tiles of
+  // 128-element rows stream under the light one (heavy: 184 against 160 us at 64 x 4096).
+  const bool cached_stream = stream_kv && (ht == 4 || D == 64);
   const bool two = two_per_simd(ht, D);
-  if (by_length && (two || (stream_kv && !heavy_stream))) wpg = kMaxWavesLight;
+  if (by_length && (two || (stream_kv && !cached_stream))) wpg = kMaxWavesLight;
   // Cached launches of two-head tiles of 16-bit 128- or 64-element rows: the light budget
   // at any walk length (measured against heavy: equal or faster on every shape from
   // 32 x 256 to 64 x 1024 and 24 x 2048, e.g. 64 x 1024 45.2 -> 42.1 us; D=64 64 x 1024
-  // 26.4 -> 23.5 us, 128 x 1024 54.1 -> 44.4 us). Four-head tiles keep the rule below
-  // (64 x 1024 with 32 / 8 heads: heavy 49.1, light 77.7 us).
+  // 26.4 -> 23.5 us, 128 x 1024 54.1 -> 44.4 us). Four-head tiles of 64-element rows, and
+  // 32-bit rows, keep the rule of grid and walk.
   const bool light_rows = ht <= 2 && (D == 128 || D == 64) && dtype != TS_F32;
-  const bool light = (stream_kv && !heavy_stream) ||
+  const bool light = two || (stream_kv && !cached_stream) ||
                      (!stream_kv && (light_rows || light_budget(grid_waves, max_blocks > 0 && walk < 512)));
   // With two waves per SIMD the chip holds twice the waves: up to 8 per workgroup, so
   // that each walks fewer tokens (fewer dependent rounds of loads per wave).
-  if (stream_kv && !by_length && !heavy_stream) {
+  if (stream_kv && !by_length && !cached_stream) {
     while (wpg < kMaxWavesLight && waves * wpg < 2 * want) wpg *= 2;
-  } else if ((light || two) && !by_length) {
+  } else if (light && !by_length) {
     while (wpg < kMaxWavesLight && waves * wpg * 2 <= 2 * want) wpg *= 2;
   }
   plan->ht = ht;
   plan->wpg = wpg;
   plan->by_length = by_length;
-  plan->budget = !light ? kHeavy : stream_kv ? kLightStream : kLight;
+  plan->budget = !light ? kHeavy : stream_kv && !cached_stream ? kLightStream : kLight;
   plan->grid = dim3(Hq / ht, by_length ? (B + 1) / 2 : B, splits);
   // LDS: one merged state per wave (two per wave for a pair); none for one-wave groups.
   plan->lds = wpg > 1 ? static_cast<size_t>((by_length ? 2 : 1) * wpg * state_slot_bytes(ht, D)) : 0;

@@ -172,12 +172,11 @@ def decode_plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, 
 def _one_split_waves(device: int, b: int, hq: int, hkv: int, d: int, block_size: int, width: int,
                      dtype: torch.dtype) -> int:  # fmt: skip
     """SIMDs the one-split launch of these sizes occupies on ``device`` (which sets the CU
-    count): its waves, over the two waves per SIMD of the light budgets and of four-head
-    tiles of 128 or more elements."""
+    count): its waves, over the two waves per SIMD of the light budgets."""
     p = decode_plan(b, hq, hkv, d, block_size, width, 1, 0, dtype)
     gx, gy, gz = p["grid"]
     waves = gx * gy * gz * int(p["waves_per_group"])
-    return waves // 2 if p["budget"] in ("light", "light_stream") or (p["head_tile"] == 4 and d >= 128) else waves
+    return waves // 2 if p["budget"] in ("light", "light_stream") else waves
 
 
 def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int,
