@@ -624,3 +624,22 @@ def test_four_head_tiles_of_128_elements(batch: int, splits: int | None, dtype: 
     g = on_gpu(c)
     out = ha.launch_paged_decode_split(*g.args(), c.scale, c.block_size, num_splits=splits)
     assert_matches(out, oracle32(c), dtype, f"{batch} sequences, {splits} splits")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,splits,width", [(40, 1, 0), (40, 1, 400), (63, 1, 400), (5, 1, 0), (70, 1, 0),
+                                                (40, 4, 0), (3, None, 0)])  # fmt: skip
+def test_four_head_tiles_of_256_elements(batch: int, splits: int | None, width: int, dtype: torch.dtype) -> None:
+    # Length pairs of four waves under the light budget (tight tables) and the heavy one
+    # (wide ones), plain workgroups of eight waves, several per CU, partials, and the policy.
+    c = decode_case([1 + (389 * i) % 500 for i in range(batch)], 32, 8, head_dim=256, dtype=dtype, seed=batch)
+    g = on_gpu(c)
+    tables = widened(g.block_tables, max(width, g.block_tables.shape[1]))
+    if splits == 1 and 33 <= batch <= 64:
+        plan = ha.decode_plan(batch, 32, 8, 256, g.block_size, tables.shape[1], 1, dtype=dtype)
+        assert (plan["by_length"], plan["waves_per_group"]) == (True, 4)
+        assert plan["budget"] == ("heavy" if width else "light")
+    out = ha.launch_paged_decode_split(g.q, g.k_cache, g.v_cache, tables, g.context_lens, c.scale, c.block_size,
+                                       num_splits=splits)  # fmt: skip
+    assert_matches(out, oracle32(c), dtype, f"{batch} sequences, {splits} splits, width {width}")

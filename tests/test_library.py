@@ -146,6 +146,17 @@ def test_decode_budget_choices(lib: ctypes.CDLL) -> None:
     assert plan(8, 16, 8, 128, 16, 256, 1, dtype=torch.float32)["budget"] == "heavy"
 
 
+def test_decode_states_fit_the_default_lds(lib: ctypes.CDLL) -> None:
+    # Dynamic LDS past 64 KiB needs a raised limit, which no kernel asks for.
+    for d in (64, 128, 256):
+        for hq, hkv in ((16, 8), (32, 8), (64, 8), (8, 8)):
+            for b in (1, 2, 17, 33, 40, 64, 65, 300):
+                for width in (4, 64, 2560):
+                    for splits in (1, 4):
+                        plan = hip_attention.decode_plan(b, hq, hkv, d, 16, width, splits)
+                        assert plan["lds_bytes"] <= 64 << 10, (b, hq, hkv, d, width, splits, plan)
+
+
 def test_policy_splits_for_small_grids(lib: ctypes.CDLL) -> None:
     # The launcher's split count with none given (sizes only; 256 CUs assumed without a
     # device): num_splits_for's count, one launch for counts up to 4 on grids of at least

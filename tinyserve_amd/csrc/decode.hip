@@ -50,13 +50,19 @@ namespace ts {
 // the second wave per SIMD hides each wave's start-up chain (lengths, block table, first
 // loads) and merge. (Tiles of four query heads of under 128 elements stream 16 bytes per lane
 // under it: short walks merge less, 8 x 128 at D = 64 6.6 us against 7.4 at 32.) Decode tiles
-// of four heads of 128 elements or more always run the light budget: at 64
+// of four heads of 128 elements or more run the light budget: at 64
 // bytes per lane an iteration was ~3000 cycles of one wave's chain, which a
 // second wave per SIMD hides (32 q / 8 kv heads bf16, us: 16 x 1024 32.7 -> 26.1, 16 x 4096
 // 85 -> 77, 48 x U[100, 5000] 116 -> 108, 64 x U[1, 2048] 58 -> 53, 128 x 4096 384 -> 371).
+// Length pairs of 256-element tiles alone keep the rule of grid and walk: eight waves' states
+// pass kMaxGroupLds, and four light waves are one per SIMD (32 / 8 heads, us, heavy -> four
+// light waves: fp32 40 x 1024 140 -> 206, 64 x 2048 360 -> 387, bf16 64 x 2048 201 -> 213; other
+// 256-element launches gain: bf16 1 x 300 25.0 -> 20.3, 16 x 1024 58 -> 44, 128 x 1024 205 ->
+// 197, fp32 16 x 4096 261 -> 215).
 // kLightStream is kLight with K/V read by non-temporal loads,
 // for decode launches larger than the last-level cache.
 constexpr bool two_per_simd(int ht, int d) { return ht == 4 && d >= 128; }
+constexpr bool always_light(int ht, int d) { return two_per_simd(ht, d) && d <= 128; }
 enum Budget { kHeavy = 0, kLight = 1, kLightStream = 2 };
 template <int B>
 struct BudgetOf {
@@ -889,7 +895,7 @@ static int launch_attend(const AttendArgs& a, dim3 grid, bool light, size_t lds,
                            dim3(kWave * a.wpg), lds, stream, a);
         return launch_status();
       }
-      if constexpr (!two_per_simd(HT, D)) {
+      if constexpr (!always_light(HT, D)) {
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kHeavy, true>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
         return launch_status();
@@ -911,7 +917,7 @@ static int launch_attend(const AttendArgs& a, dim3 grid, bool light, size_t lds,
       return launch_status();
     }
   }
-  if constexpr (PREFILL || !two_per_simd(HT, D)) {
+  if constexpr (PREFILL || !always_light(HT, D)) {
     hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kHeavy>), grid, dim3(kWave * a.wpg),
                        lds, stream, a);
     return launch_status();
@@ -1025,8 +1031,8 @@ static int tokens_per_iteration(int dtype, int D, int ht, int budget) {
   return kWave / lpt;
 }
 
-// LDS of a cut-mode workgroup: its pieces' states.
-constexpr size_t kMaxInGroupLds = 64 << 10;
+// Dynamic LDS that a workgroup's states may take (no kernel raises its limit).
+constexpr size_t kMaxGroupLds = 64 << 10;
 
 static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_blocks, int splits,
                        int head_tile, int dtype, DecodePlan* plan) {
@@ -1073,7 +1079,7 @@ static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_bl
   // budget (64 x 4096 130 -> 120 us, 64 x 8192 257 -> 233 us); two-head tiles of
   // 128-element rows stream under the light one (heavy: 184 against 160 us at 64 x 4096).
   const bool cached_stream = stream_kv && (ht == 4 || D == 64);
-  const bool two = two_per_simd(ht, D);
+  const bool two = two_per_simd(ht, D) && (always_light(ht, D) || !by_length);
   if (by_length && (two || (stream_kv && !cached_stream))) wpg = kMaxWavesLight;
   // Cached launches of two-head tiles of 16-bit 128- or 64-element rows: the light budget
   // at any walk length (measured against heavy: equal or faster on every shape from
@@ -1152,10 +1158,10 @@ extern "C" int ts_decode_split(const void* q, const void* k_cache, const void* v
     if (block_size % tokens_per_iteration(dtype, D, p.ht, p.budget)) return TS_EUNSUPPORTED;
     // (A workgroup of eight waves drops to four to fit.)
     const int per = (p.by_length ? 2 : 1) * static_cast<int>(state_slot_bytes(p.ht, D));
-    if (two_per_simd(p.ht, D) && p.wpg > kMaxWavesPerGroup && static_cast<size_t>(per) * (splits + p.wpg) > kMaxInGroupLds)
+    if (two_per_simd(p.ht, D) && p.wpg > kMaxWavesPerGroup && static_cast<size_t>(per) * (splits + p.wpg) > kMaxGroupLds)
       a.wpg = p.wpg = kMaxWavesPerGroup;
     lds = static_cast<size_t>(per) * (splits + p.wpg);
-    if (lds > kMaxInGroupLds) return TS_EUNSUPPORTED;
+    if (lds > kMaxGroupLds) return TS_EUNSUPPORTED;
     a.cuts = splits;
   }
   return dispatch_attend<false>(a, dtype, D, p.ht, p.grid, p.budget != kHeavy, lds,
