@@ -272,7 +272,12 @@ class DecodeStep:
         if rest:
             p_idx = host_ints(rest, torch.int64, dev)
             p_starts, p_qlens = ints([starts[b] for b in rest]), ints([qlens[b] for b in rest])
+            # As wide as the prompts' own contexts (a view): the prefill launch takes the width
+            # for its longest keys, and the batch's is that of any decoding sequence. One fresh
+            # 100-token prompt beside decodes at 4096 tokens: 10.9 -> 6.8 us a layer.
             p_tables, p_lens = batch.block_tables[p_idx], batch.context_lens[p_idx]
+            if len(batch.seq_slots) == len(qlens):
+                p_tables = p_tables[:, : -(-max(len(batch.seq_slots[b]) for b in rest) // bs)]
             max_q = max(qlens[b] for b in rest)
 
         def attend(i: int, q: torch.Tensor) -> torch.Tensor:
