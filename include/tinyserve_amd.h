@@ -101,7 +101,7 @@ int ts_decode_split(const void* q, const void* k_cache, const void* v_cache,
  * The launch shape ts_decode_split picks for these sizes, without launching (a query for
  * tests and benchmarks; no reference counterpart). Writes 8 ints to plan: the register
  * budget (0 heavy: one wave per SIMD; 1 light: two per SIMD; 2 light with non-temporal
- * K/V loads), waves per workgroup, 1 if workgroups take length pairs, query heads per
+ * K/V loads; 3 light at 32 bytes per lane for tiles of four heads, where 1 streams 16), waves per workgroup, 1 if workgroups take length pairs, query heads per
  * wave, the grid's x, y, z, and the dynamic LDS bytes per workgroup.
  */
 int ts_decode_plan(int B, int Hq, int Hkv, int D, int block_size, int max_blocks, int splits,

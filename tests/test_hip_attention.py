@@ -434,8 +434,8 @@ def test_paired_sequences_of_2_to_the_25_tokens() -> None:
 def test_both_register_budgets(batch: int, splits: int, heads: tuple[int, int], dtype: torch.dtype) -> None:
     # The table width bounds the tokens a wave walks; under 512 of them the kernel runs
     # its light budget (two waves per SIMD, up to 8 a workgroup), else, for fp32 at two
-    # heads a wave, the heavy one. (16-bit two-head tiles and four-head tiles of 128
-    # elements are light at any walk.) The same sequences through their own narrow table
+    # heads a wave, the heavy one. (16-bit two-head tiles are light at any walk; four-head
+    # tiles of 128 elements are too, at 32 bytes a lane where walks are long.) The same sequences through their own narrow table
     # and through one widened to 2000 blocks give the reference either way: length pairs
     # (64, 45), in-workgroup splits (32 x 4), a small batch, and HBM splits with the combine
     # (8 x 8), at GQA groups of 2 and 4.
@@ -520,8 +520,8 @@ def test_streaming_launches(dtype: torch.dtype, head_dim: int, heads: tuple[int,
     for splits in (1, 4):
         plan = ha.decode_plan(b, *heads, head_dim, g.block_size, 8192, splits, head_tile, dtype)
         # Rows of 64 elements run the heavy budget and tiles of four query heads of 128 the
-        # light one, both with cached loads; the others stream.
-        cached = "heavy" if head_dim == 64 else "light" if plan["head_tile"] == 4 else None
+        # light one at 32 bytes a lane, both with cached loads; the others stream.
+        cached = "heavy" if head_dim == 64 else "light_wide" if plan["head_tile"] == 4 else None
         assert plan["budget"] == (cached or "light_stream"), plan
         tight = ha._launch(*g.args(), g.scale, g.block_size, splits, head_tile)
         out = ha._launch(g.q, g.k_cache, g.v_cache, wide, g.context_lens, g.scale, g.block_size, splits,
@@ -643,3 +643,24 @@ def test_four_head_tiles_of_256_elements(batch: int, splits: int | None, width: 
     out = ha.launch_paged_decode_split(g.q, g.k_cache, g.v_cache, tables, g.context_lens, c.scale, c.block_size,
                                        num_splits=splits)  # fmt: skip
     assert_matches(out, oracle32(c), dtype, f"{batch} sequences, {splits} splits, width {width}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("batch,head_dim,longest,splits", [(2, 128, 30, 1), (40, 128, 16, 1), (220, 128, 30, 1),
+                                                           (64, 128, 90, 4), (300, 128, 60, 16), (220, 256, 16, 1),
+                                                           (64, 256, 40, 4)])  # fmt: skip
+def test_short_walks_of_four_head_tiles(batch: int, head_dim: int, longest: int, splits: int,
+                                        dtype: torch.dtype) -> None:  # fmt: skip
+    # Walks of few bytes per wave: 16 bytes a lane where a wave has under 8 to 32 KB of K (fp16
+    # here, and fp32 over several rounds), in workgroups of eight waves, length pairs, lone
+    # waves, cut into ranges inside the workgroup and as partials.
+    c = decode_case([1 + (7 * i) % longest for i in range(batch)], 32, 8, head_dim=head_dim, dtype=dtype, seed=batch)
+    g = on_gpu(c)
+    tables = g.block_tables[:, : -(-longest // c.block_size)]
+    plan = ha.decode_plan(batch, 32, 8, head_dim, c.block_size, tables.shape[1], 1, dtype=dtype)
+    if dtype == torch.float16 and head_dim == 128 and splits == 1:
+        assert plan["budget"] == "light", plan
+    out = ha.launch_paged_decode_split(g.q, g.k_cache, g.v_cache, tables, g.context_lens, c.scale, c.block_size,
+                                       num_splits=splits)  # fmt: skip
+    assert_matches(out, oracle32(c), dtype, f"{batch} sequences, {splits} splits, D={head_dim}")

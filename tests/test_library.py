@@ -131,17 +131,18 @@ def test_decode_budget_choices(lib: ctypes.CDLL) -> None:
     # Which register budget a launch runs (sizes only). Streaming launches (K/V bounded by
     # the table width above 256 MiB): light-stream for two-head tiles of 128-element rows,
     # cached loads under the heavy budget for 64-element rows. Four-head tiles of 128
-    # elements: light, cached, always. Cached launches of two-head 16-bit tiles: light at any
-    # walk length; fp32 keeps the walk rule (heavy for long walks on one round of waves).
+    # elements: light at 32 bytes a lane, cached, but for short walks. Cached launches of
+    # two-head 16-bit tiles: light at any walk length; fp32 keeps the walk rule (heavy for
+    # long walks on one round of waves).
     plan = hip_attention.decode_plan
     assert plan(64, 16, 8, 128, 16, 256, 1)["budget"] == "light_stream"
-    assert plan(64, 32, 8, 128, 16, 256, 1)["budget"] == "light"  # four-head tiles
+    assert plan(64, 32, 8, 128, 16, 256, 1)["budget"] == "light_wide"  # four-head tiles
     assert plan(64, 32, 8, 128, 16, 256, 1)["head_tile"] == 4
     assert plan(64, 16, 8, 64, 16, 512, 1)["budget"] == "heavy"  # D=64, 512 MiB bound
     assert plan(64, 16, 8, 128, 16, 64, 1)["budget"] == "light"  # 64 x 1024, cached
     assert plan(16, 16, 8, 128, 16, 128, 1, dtype=torch.bfloat16)["budget"] == "light"
     assert plan(64, 16, 8, 64, 16, 64, 1)["budget"] == "light"  # D=64, cached
-    assert plan(64, 32, 8, 128, 16, 64, 1)["budget"] == "light"  # four heads, long walks
+    assert plan(64, 32, 8, 128, 16, 64, 1)["budget"] == "light_wide"  # four heads, long walks
     assert plan(64, 32, 8, 64, 16, 64, 1, dtype=torch.float32)["budget"] == "heavy"  # four of 64
     assert plan(8, 16, 8, 128, 16, 256, 1, dtype=torch.float32)["budget"] == "heavy"
 
@@ -155,6 +156,22 @@ def test_decode_states_fit_the_default_lds(lib: ctypes.CDLL) -> None:
                     for splits in (1, 4):
                         plan = hip_attention.decode_plan(b, hq, hkv, d, 16, width, splits)
                         assert plan["lds_bytes"] <= 64 << 10, (b, hq, hkv, d, width, splits, plan)
+
+
+def test_wide_budget_of_four_head_tiles(lib: ctypes.CDLL) -> None:
+    # Bytes of K per wave, both sides of each line: 8 KB for workgroups of several waves,
+    # 16 KB (fp32 8) for lone waves in one round, 32 KB in several; never 256-element pairs.
+    def budget(b: int, d: int, width: int, splits: int = 1, dtype: torch.dtype = torch.float16) -> str:
+        return hip_attention.decode_plan(b, 32, 8, d, 16, width, splits, dtype=dtype)["budget"]
+
+    assert budget(4, 128, 8) == "light" and budget(4, 128, 9) == "light_wide"  # eight waves: 16, 32 tokens
+    assert budget(4, 128, 1, dtype=torch.float32) == "light_wide" == budget(4, 256, 1)
+    assert budget(200, 128, 3) == "light" and budget(200, 128, 4) == "light_wide"  # 1600 lone waves
+    assert budget(200, 128, 1, dtype=torch.float32) == "light_wide"
+    assert budget(100, 128, 28, 4) == "light" and budget(100, 128, 29, 4) == "light_wide"  # 3200
+    assert budget(300, 128, 100) == "light_wide"
+    assert budget(40, 256, 4) == "light" and budget(40, 256, 256) == "heavy"
+    assert budget(24, 256, 256) == "light_wide"
 
 
 def test_policy_splits_for_small_grids(lib: ctypes.CDLL) -> None:

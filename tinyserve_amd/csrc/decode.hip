@@ -48,22 +48,12 @@ namespace ts {
 // waves all run in one round, where each wave must keep much in flight. kLight: 32 bytes
 // per lane, two in flight, two waves per SIMD -- for launches of several rounds, where
 // the second wave per SIMD hides each wave's start-up chain (lengths, block table, first
-// loads) and merge. (Tiles of four query heads of under 128 elements stream 16 bytes per lane
-// under it: short walks merge less, 8 x 128 at D = 64 6.6 us against 7.4 at 32.) Decode tiles
-// of four heads of 128 elements or more run the light budget: at 64
-// bytes per lane an iteration was ~3000 cycles of one wave's chain, which a
-// second wave per SIMD hides (32 q / 8 kv heads bf16, us: 16 x 1024 32.7 -> 26.1, 16 x 4096
-// 85 -> 77, 48 x U[100, 5000] 116 -> 108, 64 x U[1, 2048] 58 -> 53, 128 x 4096 384 -> 371).
-// Length pairs of 256-element tiles alone keep the rule of grid and walk: eight waves' states
-// pass kMaxGroupLds, and four light waves are one per SIMD (32 / 8 heads, us, heavy -> four
-// light waves: fp32 40 x 1024 140 -> 206, 64 x 2048 360 -> 387, bf16 64 x 2048 201 -> 213; other
-// 256-element launches gain: bf16 1 x 300 25.0 -> 20.3, 16 x 1024 58 -> 44, 128 x 1024 205 ->
-// 197, fp32 16 x 4096 261 -> 215).
-// kLightStream is kLight with K/V read by non-temporal loads,
-// for decode launches larger than the last-level cache.
-constexpr bool two_per_simd(int ht, int d) { return ht == 4 && d >= 128; }
-constexpr bool always_light(int ht, int d) { return two_per_simd(ht, d) && d <= 128; }
-enum Budget { kHeavy = 0, kLight = 1, kLightStream = 2 };
+// loads) and merge. (Tiles of four query heads stream 16 bytes per lane under it: short
+// walks merge less.) kLightStream is kLight with K/V read by non-temporal loads, for decode
+// launches larger than the last-level cache. kLightWide: kLight at 32 bytes per lane, for
+// decode tiles of four heads of 128 elements or more with long walks (wide_tiles).
+enum Budget { kHeavy = 0, kLight = 1, kLightStream = 2, kLightWide = 3 };
+constexpr bool has_wide(int ht, int d) { return ht == 4 && d >= 128; }
 template <int B>
 struct BudgetOf {
   static constexpr bool kLightish = B != kHeavy;
@@ -110,7 +100,6 @@ struct AttendArgs {
   int nseq;       // decode: sequences in the batch
   int64_t q_sb, q_sh, o_sb, o_sh, k_ss, k_sh, bt_s;
   float scale_log2;  // softmax scale * log2(e)
-  int stream_kv;     // decode, light budget: K/V through non-temporal loads
   // decode, in-workgroup split-K: the walk of each sequence is cut at the block ranges of
   // `cuts` splits (split s: blocks [s * ceil(n / cuts), ...), the reference's ranges);
   // every range piece's softmax state is parked in LDS and the workgroup merges them. 0:
@@ -362,7 +351,10 @@ template <typename T, int D, int HT, bool PREFILL, int BUDGET, bool CUT = false>
 __global__ __launch_bounds__(PREFILL ? kWave : kWave * (BudgetOf<BUDGET>::kLightish ? kMaxWavesLight : kMaxWavesPerGroup))
 __attribute__((amdgpu_waves_per_eu(BudgetOf<BUDGET>::kWavesPerEU)))
 void paged_attend_kernel(const AttendArgs a) {
-  constexpr int LB = BudgetOf<BUDGET>::kLightish && HT == 4 && D < 128 ? 16 : BudgetOf<BUDGET>::kLaneBytes;
+  // Tiles of four heads stream 16 bytes per lane under kLight; the generic prefill's rows of
+  // 128 elements or more 32 (32 / 8 heads, us, 16 -> 32 bytes: fp32 4 x 256 177 -> 145, 2 x
+  // (700 cached + 200) 374 -> 284, D = 256 fp16 4 x 256 242 -> 199).
+  constexpr int LB = BUDGET == kLight && HT == 4 && (!PREFILL || D < 128) ? 16 : BudgetOf<BUDGET>::kLaneBytes;
   using S = RowShape<T, D, LB>;
   constexpr int LPT = S::kLPT, NV = S::kNV, VEC = S::kVec, TPW = S::kTPW, E = S::kE;
   // Streaming launches are bound by issue, cached ones (short walks) by latency.
@@ -879,60 +871,68 @@ __global__ __launch_bounds__(64) void combine_kernel(const float* __restrict__ m
 }
 
 template <typename T, int D, int HT, bool PREFILL>
-static int launch_attend(const AttendArgs& a, dim3 grid, bool light, size_t lds, hipStream_t stream) {
+static int launch_attend(const AttendArgs& a, dim3 grid, int budget, size_t lds, hipStream_t stream) {
   if constexpr (!PREFILL) {
     if (a.cuts > 1) {
       // In-workgroup split-K over the reference's split ranges (cut mode).
+      if constexpr (has_wide(HT, D)) {
+        if (budget == kLightWide) {
+          hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kLightWide, true>), grid,
+                             dim3(kWave * a.wpg), lds, stream, a);
+          return launch_status();
+        }
+      }
       if constexpr (HT < 4 && (D == 64 || D == 128)) {
-        if (light && a.stream_kv) {
+        if (budget == kLightStream) {
           hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kLightStream, true>), grid,
                              dim3(kWave * a.wpg), lds, stream, a);
           return launch_status();
         }
       }
-      if (light) {
+      if (budget != kHeavy) {
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kLight, true>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
         return launch_status();
       }
-      if constexpr (!always_light(HT, D)) {
-        hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kHeavy, true>), grid,
-                           dim3(kWave * a.wpg), lds, stream, a);
-        return launch_status();
-      }
-      return TS_EUNSUPPORTED;  // the plan gives these tiles the light budget
+      hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, false, kHeavy, true>), grid,
+                         dim3(kWave * a.wpg), lds, stream, a);
+      return launch_status();
     }
   }
   {
+    if constexpr (!PREFILL && has_wide(HT, D)) {
+      if (budget == kLightWide) {
+        hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kLightWide>), grid,
+                           dim3(kWave * a.wpg), lds, stream, a);
+        return launch_status();
+      }
+    }
     if constexpr (!PREFILL && HT < 4 && (D == 64 || D == 128)) {
-      if (light && a.stream_kv) {
+      if (budget == kLightStream) {
         hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kLightStream>), grid,
                            dim3(kWave * a.wpg), lds, stream, a);
         return launch_status();
       }
     }
-    if (light) {
+    if (budget != kHeavy) {
       hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kLight>), grid,
                          dim3(kWave * a.wpg), lds, stream, a);
       return launch_status();
     }
   }
-  if constexpr (PREFILL || !always_light(HT, D)) {
-    hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kHeavy>), grid, dim3(kWave * a.wpg),
-                       lds, stream, a);
-    return launch_status();
-  }
-  return TS_EUNSUPPORTED;  // the plan gives these tiles the light budget
+  hipLaunchKernelGGL((paged_attend_kernel<T, D, HT, PREFILL, kHeavy>), grid, dim3(kWave * a.wpg),
+                     lds, stream, a);
+  return launch_status();
 }
 
 template <typename T, bool PREFILL>
-static int dispatch_d(const AttendArgs& a, int D, int ht, dim3 grid, bool light, size_t lds,
+static int dispatch_d(const AttendArgs& a, int D, int ht, dim3 grid, int budget, size_t lds,
                       hipStream_t stream) {
 #define TS_HT(DD)                                                                \
   switch (ht) {                                                                  \
-    case 1: return launch_attend<T, DD, 1, PREFILL>(a, grid, light, lds, stream); \
-    case 2: return launch_attend<T, DD, 2, PREFILL>(a, grid, light, lds, stream); \
-    case 4: return launch_attend<T, DD, 4, PREFILL>(a, grid, light, lds, stream); \
+    case 1: return launch_attend<T, DD, 1, PREFILL>(a, grid, budget, lds, stream); \
+    case 2: return launch_attend<T, DD, 2, PREFILL>(a, grid, budget, lds, stream); \
+    case 4: return launch_attend<T, DD, 4, PREFILL>(a, grid, budget, lds, stream); \
     default: return TS_EUNSUPPORTED;                                             \
   }
   switch (D) {
@@ -956,11 +956,11 @@ static bool light_budget(int64_t waves, bool short_walks) {
 
 template <bool PREFILL>
 static int dispatch_attend(const AttendArgs& a, int dtype, int D, int ht, dim3 grid,
-                           bool light, size_t lds, hipStream_t stream) {
+                           int budget, size_t lds, hipStream_t stream) {
   switch (dtype) {
-    case TS_F32: return dispatch_d<float, PREFILL>(a, D, ht, grid, light, lds, stream);
-    case TS_F16: return dispatch_d<f16, PREFILL>(a, D, ht, grid, light, lds, stream);
-    case TS_BF16: return dispatch_d<bf16, PREFILL>(a, D, ht, grid, light, lds, stream);
+    case TS_F32: return dispatch_d<float, PREFILL>(a, D, ht, grid, budget, lds, stream);
+    case TS_F16: return dispatch_d<f16, PREFILL>(a, D, ht, grid, budget, lds, stream);
+    case TS_BF16: return dispatch_d<bf16, PREFILL>(a, D, ht, grid, budget, lds, stream);
     default: return TS_EUNSUPPORTED;
   }
 }
@@ -989,7 +989,7 @@ int prefill_rows_generic(const void* q, const void* k, const void* v, void* out,
                scale * kLog2e};
   dim3 grid(static_cast<unsigned>(R) * max_q_len, Hq / ht, 1);
   const int64_t waves = static_cast<int64_t>(grid.x) * grid.y;
-  return dispatch_attend<true>(a, dtype, D, ht, grid, light_budget(waves, false), 0, stream);
+  return dispatch_attend<true>(a, dtype, D, ht, grid, light_budget(waves, false) ? kLight : kHeavy, 0, stream);
 }
 
 template <typename T>
@@ -1018,14 +1018,14 @@ struct DecodePlan {
   int ht;         // query heads per wave
   int wpg;        // waves per workgroup
   int by_length;  // workgroups take length pairs
-  int budget;     // kHeavy, kLight or kLightStream
+  int budget;     // a Budget
   dim3 grid;
   size_t lds;     // dynamic LDS bytes
 };
 
 // Tokens one wave streams per loop iteration (TPW of the kernel's RowShape).
 static int tokens_per_iteration(int dtype, int D, int ht, int budget) {
-  const int lb = budget == kHeavy ? 64 : ht == 4 && D < 128 ? 16 : 32;
+  const int lb = budget == kHeavy ? 64 : budget == kLight && ht == 4 ? 16 : 32;
   const int row = D * (dtype == TS_F32 ? 4 : 2);
   const int lpt = row <= lb ? 1 : std::min(row / lb, kWave);
   return kWave / lpt;
@@ -1033,6 +1033,29 @@ static int tokens_per_iteration(int dtype, int D, int ht, int budget) {
 
 // Dynamic LDS that a workgroup's states may take (no kernel raises its limit).
 constexpr size_t kMaxGroupLds = 64 << 10;
+
+// Whether tiles of four heads of 128 elements or more run kLightWide (`groups` workgroups of wpg
+// waves) in place of what the rules of the other tiles give: heavy, or light with each wave
+// walking at most `tokens`. Against heavy, whose iteration of 64 bytes per lane is ~3000
+// cycles of one wave's chain, a second wave per SIMD hides it (us: 16 x 4096 bf16 at 32 / 8
+// heads 85 -> 77, 128 x 4096 384 -> 371). Lone waves, one to 1.4 per SIMD, gain at equal
+// lengths (284 x 557 at 16 / 4 110 -> 83, mean ratio 0.77) and not on ragged ones (mean 1.03, 77
+// of U[1, 1988] at 64 / 8 175 -> 219: most run alone and wait for the SIMDs that hold two); the
+// lengths are not known here.
+// Against light at 16 bytes a walk has half the iterations, but the merge over token lanes
+// costs more, which short walks do not earn back (213 x 11 tokens bf16 9.5 -> 15.7, 253 x U[1,
+// 493] in 16 ranges 53 -> 68). The lines, in bytes of K per wave: 8 KB for workgroups of several
+// waves (mean ratio 1.01 at 4 KB, 0.94 at 8), 16 KB for lone waves in one round (1.05 at 12,
+// 0.95 at 16; fp32 0.94 at 8), 32 KB in several rounds (1.01 at 16-32, 0.86 above).
+// Over 1700 drawn batches of 4 to 64 query heads: 0.88 of the time without it.
+static bool wide_tiles(bool light, int D, int dtype, int64_t groups, int wpg, int64_t tokens) {
+  if (!light) return true;
+  const int64_t waves = groups * wpg;
+  const int64_t bytes = tokens * D * (dtype == TS_F32 ? 4 : 2);
+  if (wpg > 1) return bytes >= 8 << 10;
+  if (waves > 8 * static_cast<int64_t>(compute_units())) return bytes >= 32 << 10;
+  return bytes >= (dtype == TS_F32 ? 8 : 16) << 10;
+}
 
 static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_blocks, int splits,
                        int head_tile, int dtype, DecodePlan* plan) {
@@ -1079,27 +1102,40 @@ static int plan_decode(int B, int Hq, int Hkv, int D, int block_size, int max_bl
   // budget (64 x 4096 130 -> 120 us, 64 x 8192 257 -> 233 us); two-head tiles of
   // 128-element rows stream under the light one (heavy: 184 against 160 us at 64 x 4096).
   const bool cached_stream = stream_kv && (ht == 4 || D == 64);
-  const bool two = two_per_simd(ht, D) && (always_light(ht, D) || !by_length);
-  if (by_length && (two || (stream_kv && !cached_stream))) wpg = kMaxWavesLight;
+  if (by_length && stream_kv && !cached_stream) wpg = kMaxWavesLight;
   // Cached launches of two-head tiles of 16-bit 128- or 64-element rows: the light budget
   // at any walk length (measured against heavy: equal or faster on every shape from
   // 32 x 256 to 64 x 1024 and 24 x 2048, e.g. 64 x 1024 45.2 -> 42.1 us; D=64 64 x 1024
   // 26.4 -> 23.5 us, 128 x 1024 54.1 -> 44.4 us). Four-head tiles of 64-element rows, and
   // 32-bit rows, keep the rule of grid and walk.
   const bool light_rows = ht <= 2 && (D == 128 || D == 64) && dtype != TS_F32;
-  const bool light = two || (stream_kv && !cached_stream) ||
+  const bool light = (stream_kv && !cached_stream) ||
                      (!stream_kv && (light_rows || light_budget(grid_waves, max_blocks > 0 && walk < 512)));
   // With two waves per SIMD the chip holds twice the waves: up to 8 per workgroup, so
   // that each walks fewer tokens (fewer dependent rounds of loads per wave).
+  int light_wpg = wpg;
   if (stream_kv && !by_length && !cached_stream) {
-    while (wpg < kMaxWavesLight && waves * wpg < 2 * want) wpg *= 2;
-  } else if (light && !by_length) {
-    while (wpg < kMaxWavesLight && waves * wpg * 2 <= 2 * want) wpg *= 2;
+    while (light_wpg < kMaxWavesLight && waves * light_wpg < 2 * want) light_wpg *= 2;
+  } else if (!by_length) {
+    while (light_wpg < kMaxWavesLight && waves * light_wpg * 2 <= 2 * want) light_wpg *= 2;
   }
+  // Length pairs of 256-element tiles keep heavy or light: eight wide waves' states pass
+  // kMaxGroupLds, and four are one per SIMD (32 / 8 heads, us, heavy -> four wide: fp32 40 x
+  // 1024 140 -> 206, 64 x 2048 360 -> 387, bf16 64 x 2048 201 -> 213).
+  bool wide = false;
+  if (has_wide(ht, D) && (!by_length || D == 128)) {
+    const int wide_wpg = by_length ? kMaxWavesLight : light_wpg;
+    const int64_t range = by_length ? 2 * static_cast<int64_t>(max_blocks) : (max_blocks + splits - 1) / splits;
+    const int64_t blocks = (range + light_wpg - 1) / light_wpg;  // of a wave under the light budget
+    wide = wide_tiles(light, D, dtype, static_cast<int64_t>(Hq / ht) * (by_length ? (B + 1) / 2 : B) * splits,
+                      wide_wpg, blocks * block_size);
+    if (wide) wpg = wide_wpg;
+  }
+  if (light && !wide) wpg = light_wpg;
   plan->ht = ht;
   plan->wpg = wpg;
   plan->by_length = by_length;
-  plan->budget = !light ? kHeavy : stream_kv && !cached_stream ? kLightStream : kLight;
+  plan->budget = wide ? kLightWide : !light ? kHeavy : stream_kv ? kLightStream : kLight;
   plan->grid = dim3(Hq / ht, by_length ? (B + 1) / 2 : B, splits);
   // LDS: one merged state per wave (two per wave for a pair); none for one-wave groups.
   plan->lds = wpg > 1 ? static_cast<size_t>((by_length ? 2 : 1) * wpg * state_slot_bytes(ht, D)) : 0;
@@ -1148,8 +1184,7 @@ extern "C" int ts_decode_split(const void* q, const void* k_cache, const void* v
   AttendArgs a{q, k_cache, v_cache, block_tables, context_lens, out, m, l, acc, nullptr,
                nullptr, Hq, Hq / Hkv, ilog2(block_size), in_group ? 1 : splits, p.wpg, 0,
                p.by_length, B, q_stride_b, q_stride_h, o_stride_b, o_stride_h, k_stride_slot,
-               k_stride_head, bt_stride, scale * kLog2e, 0};
-  a.stream_kv = p.budget == kLightStream ? 1 : 0;
+               k_stride_head, bt_stride, scale * kLog2e};
   a.width = max_blocks > 0 && max_blocks <= kWave && !p.by_length ? max_blocks : 0;
   size_t lds = p.lds;
   if (in_group) {
@@ -1158,13 +1193,13 @@ extern "C" int ts_decode_split(const void* q, const void* k_cache, const void* v
     if (block_size % tokens_per_iteration(dtype, D, p.ht, p.budget)) return TS_EUNSUPPORTED;
     // (A workgroup of eight waves drops to four to fit.)
     const int per = (p.by_length ? 2 : 1) * static_cast<int>(state_slot_bytes(p.ht, D));
-    if (two_per_simd(p.ht, D) && p.wpg > kMaxWavesPerGroup && static_cast<size_t>(per) * (splits + p.wpg) > kMaxGroupLds)
+    if (has_wide(p.ht, D) && p.wpg > kMaxWavesPerGroup && static_cast<size_t>(per) * (splits + p.wpg) > kMaxGroupLds)
       a.wpg = p.wpg = kMaxWavesPerGroup;
     lds = static_cast<size_t>(per) * (splits + p.wpg);
     if (lds > kMaxGroupLds) return TS_EUNSUPPORTED;
     a.cuts = splits;
   }
-  return dispatch_attend<false>(a, dtype, D, p.ht, p.grid, p.budget != kHeavy, lds,
+  return dispatch_attend<false>(a, dtype, D, p.ht, p.grid, p.budget, lds,
                                 static_cast<hipStream_t>(stream));
 }
 

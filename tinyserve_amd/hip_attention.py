@@ -151,7 +151,7 @@ def num_splits_for(
     return max(1, min(want, MAX_SPLITS, max_blocks))
 
 
-BUDGETS = ("heavy", "light", "light_stream")
+BUDGETS = ("heavy", "light", "light_stream", "light_wide")
 
 
 def decode_plan(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int,
@@ -176,7 +176,7 @@ def _one_split_waves(device: int, b: int, hq: int, hkv: int, d: int, block_size:
     p = decode_plan(b, hq, hkv, d, block_size, width, 1, 0, dtype)
     gx, gy, gz = p["grid"]
     waves = gx * gy * gz * int(p["waves_per_group"])
-    return waves // 2 if p["budget"] in ("light", "light_stream") else waves
+    return waves if p["budget"] == "heavy" else waves // 2
 
 
 def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int, block_size: int,
