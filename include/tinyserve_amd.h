@@ -183,6 +183,13 @@ int ts_prefill_varlen_ws(const void* q, const void* k_cache, const void* v_cache
 int64_t ts_prefill_workspace(int R, int Hq, int Hkv, int D, int block_size, int max_q_len,
                              int64_t max_keys, int dtype);
 
+/* The workgroup shape ts_prefill_varlen_ws runs for these sizes, its workspace given and rows
+ * 16-byte aligned (a query for tests and benchmarks; no reference counterpart): 0 one wave per
+ * row; 1 eight waves, 64-key tiles; 2 keys split in two halves; 3 four waves, 32-key tiles;
+ * keys cut over workgroups of 4 eight waves, 5 two halves. Negative: TS_EINVAL. */
+int ts_prefill_plan(int R, int Hq, int Hkv, int D, int block_size, int max_q_len, int64_t n_rows,
+                    int64_t max_keys, int dtype);
+
 /*
  * RMSNorm of every row of x [T, N]:
  *   out = (T)(x * 1/sqrt(mean(x^2) + eps)) * w   (normalise in fp32, multiply in T)

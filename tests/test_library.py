@@ -227,6 +227,26 @@ def test_policy_runs_short_tables_as_one_launch(lib: ctypes.CDLL) -> None:
         assert hip_attention.policy_splits(4, hq, 8, 128, 16, line + 1) > 1
 
 
+@pytest.mark.parametrize(("heads", "specs", "want"), [
+    # (cached, new) tokens: fresh prompts, one round of the key-split shape's workgroups and more;
+    ((16, 8, 128), [(0, 64)], "short_tiles"), ((16, 8, 128), [(0, 128)] * 8, "short_tiles"),
+    ((16, 8, 128), [(0, 200)] * 16, "short_tiles"), ((16, 8, 128), [(0, 512)], "key_split"),
+    ((16, 8, 128), [(0, 512)] * 8, "short_tiles"), ((16, 8, 128), [(0, 2048)], "key_split"),
+    ((16, 8, 128), [(0, 2048)] * 2, "key_split"), ((16, 8, 128), [(0, 2048)] * 4, "short_tiles"),
+    ((16, 8, 128), [(0, 1408)] * 24, "eight_wave"),
+    # chunks of few new tokens behind cached ones: their walk is long all the same;
+    ((16, 8, 128), [(629, 219)] * 5, "key_split"), ((32, 8, 128), [(800, 160)] * 3, "key_split"),
+    ((8, 8, 128), [(2697, 403), (0, 403)] * 5, "key_split"), ((16, 8, 128), [(2849, 143)] * 25, "short_tiles"),
+    ((16, 8, 128), [(200, 100)] * 4, "eight_wave"), ((64, 8, 128), [(0, 100)], "eight_wave"),
+    ((16, 8, 256), [(0, 100)], "rows"),
+])  # fmt: skip
+def test_prefill_shape_choices(lib: ctypes.CDLL, heads: tuple[int, int, int], specs: list[tuple[int, int]],
+                               want: str) -> None:  # fmt: skip
+    new = [n for _, n in specs]
+    keys = -(-max(c + n for c, n in specs) // 16) * 16
+    assert hip_prefill.prefill_plan(len(specs), *heads, 16, max(new), sum(new), keys) == want
+
+
 # --- decode entry points: the reference's argument errors (test_triton_attention.py:201-234)
 
 

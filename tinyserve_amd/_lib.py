@@ -59,6 +59,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _f, _i, _i64, _vp, _i64, _vp],  # scale dtype max_keys workspace floats stream
     ),
     "ts_prefill_workspace": (_i64, [_i, _i, _i, _i, _i, _i, _i64, _i]),
+    "ts_prefill_plan": (_i, [_i, _i, _i, _i, _i, _i, _i64, _i64, _i]),
     "ts_rms_norm_rows": (_i, [_vp, _vp, _vp, _i, _i, _i64, _i64, _f, _i, _vp]),
     "ts_add_rms_norm_rows": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i64, _i64, _i64, _f, _i, _vp]),
     "ts_silu_mul": (_i, [_vp, _vp, _i, _i, _i64, _i64, _i, _vp]),

@@ -1051,21 +1051,26 @@ static int dispatch_hg_w(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows,
 // Which of the three workgroup shapes a launch runs (see the header comment). wg8 is the
 // 8-wave grid, n4 the key-split shape's workgroups with query tiles in them (counted from
 // the rows where the host knows them: a grid sized by the longest of mixed prompts is mostly
-// empty), max_keys a bound on every context (0: unknown). The key-split shape runs one
-// workgroup per CU: it wins while one round holds them all, and in two rounds only on long
-// walks; the 4-wave, 32-key shape (three per CU) takes what is left of the small and
-// mid-size launches. Measured, us (16 q / 8 kv heads, D = 128, fp16, key-split / 32-key /
-// 8-wave): 1 x 64 7.3 / 5.7 / 5.6, 8 x 128 8.8 / 7.5 / 8.9, 1 x 512 12.7 / 14.2 / 16.7,
-// 4 x 512 14.7 / 15.9 / 18.2, 8 x 512 23.4 / 19.8 / 21.7, 16 x 200 19.0 / 14.1 / 14.0, six
-// prompts of 355-576 20.3 / 18.4 / 19.4, three of up to 2294 36.2 / 49.0 / 56.7, 2 x 2048
-// 45.8 / 51.8 / 55.8; 32 / 8 heads: 5 x 300 17.7 / 12.6 / 13.9, 3 x 700 30.4 / 23.3 / 24.2,
-// 1 x 1024 20.4 / 23.9 / 28.8. Grids of up to 8 8-wave workgroups per CU (3-16 prompts of
-// 2048, 1-4 of 4096-8192: +1-10%), and of up to 16 when the mean new tokens per sequence is
-// at most 1280 (8-32 mixed prompts: +5-14%), the 32-key shape; larger grids the 8-wave one.
+// empty), max_keys a bound on every context (0: unknown, taken for long). The key-split shape
+// runs one workgroup per CU and halves the longest walk; the 4-wave, 32-key shape (three per
+// CU) starts and ends sooner, and takes what is left of the small and mid-size launches. So
+// the key-split one wins from a walk on (keys a query of the longest sequence sees, cached
+// ones included) that grows with the rounds of n4: 250 keys times their square, and 150 at
+// least. Measured, us (16 q / 8 kv heads, D = 128, fp16, key-split / 32-key / 8-wave): 1 x 512
+// 12.7 / 14.2 / 16.7, 8 x 512 23.4 / 19.8 / 21.7, 16 x 200 19.0 / 14.1 / 14.0, six prompts of
+// 355-576 20.3 / 18.4 / 19.4, three of up to 2294 36.2 / 49.0 / 56.7, 2 x 2048 45.8 / 51.8 /
+// 55.8; behind cached keys (cached + new, bf16) 1 x (14474 + 214) 235 / 372 / 439, 5 x (629 +
+// 219) 23.3 / 28.6 / 33.5, 25 x (2849 + 143) 68 / 57 / 66. Over 920 drawn batches that the line
+// decides: 1.2% over the better shape of each; two lose over 5% against the key-split shape
+// throughout (the most 14%). By the new tokens alone, without the cached keys, up to 58% were
+// lost. Up to 128 new tokens without a long prefix (8 tiles of 32 keys): 1 x 64 7.3 / 5.7 / 5.6,
+// 8 x 128 8.8 / 7.5 / 8.9, 47 x (U[123, 247] + U[1, 10]) 32-key 14.0, 8-wave 20.7. Grids of up to 8
+// 8-wave workgroups per CU (3-16 prompts of 2048, 1-4 of 4096-8192: +1-10%), and of up to 16
+// when the mean new tokens per sequence is at most 1280 (8-32 mixed prompts: +5-14%), the
+// 32-key shape; larger grids the 8-wave one.
 enum class PrefillShape { kW8, kW4, kW4Short };
 
-static PrefillShape prefill_shape(int R, int group, int Hkv, int D, int max_q_len, int64_t n_rows,
-                                  int64_t max_keys) {
+static PrefillShape prefill_shape(int R, int group, int Hkv, int max_q_len, int64_t n_rows, int64_t max_keys) {
   const int hg8 = group < 8 ? group : 8;
   const int64_t wg8 = static_cast<int64_t>((max_q_len + 32 * (8 / hg8) - 1) / (32 * (8 / hg8))) *
                       R * Hkv * (group / hg8);
@@ -1084,9 +1089,9 @@ static PrefillShape prefill_shape(int R, int group, int Hkv, int D, int max_q_le
   const int64_t longest = static_cast<int64_t>(R) * ((max_q_len + oq - 1) / oq);
   const bool mixed = n_rows > 0 && n_rows < static_cast<int64_t>(R) * max_q_len;
   const int64_t n4 = Hkv * (mixed ? std::min(longest, n_rows / oq + (R + 1) / 2) : longest);
-  const int64_t mean = mixed ? n_rows / R : max_q_len;
-  const bool one_round = 100 * n4 <= (D == 64 ? 115 : 110) * cus;
-  if (one_round ? mean >= (D == 64 ? 100 : 224) : max_q_len * cus >= 1000 * n4) return PrefillShape::kW4;
+  const int64_t past = max_keys > 0 ? std::max<int64_t>(max_keys - max_q_len, 0) : int64_t{1} << 31;
+  const int64_t walk = past + max_q_len / 2;
+  if (2 * wg8 < 3 * cus && walk >= 150 && walk * cus * cus >= 250 * n4 * n4) return PrefillShape::kW4;
   const bool short_mean = n_rows > 0 && n_rows <= 1280 * static_cast<int64_t>(R);
   if (wg8 <= 8 * cus || (short_mean && wg8 <= 16 * cus)) return PrefillShape::kW4Short;
   return PrefillShape::kW8;
@@ -1124,7 +1129,7 @@ static bool cut_shape(int R, int group, int Hkv, int D, int lbs, int max_q_len, 
   if (items > kWave) return false;
   // What a cut can gain, in steps of the longest workgroup of the shape that runs
   // otherwise (`fill`: its workgroups per CU).
-  const bool halves = prefill_shape(R, group, Hkv, D, max_q_len, 0, max_keys) == PrefillShape::kW4;
+  const bool halves = prefill_shape(R, group, Hkv, max_q_len, 0, max_keys) == PrefillShape::kW4;
   if (!halves && max_q_len > 128) return false;
   const int hg = halves ? std::min(group, 4) : std::min(group, 8);
   const int oq = 32 * ((halves ? 4 : 8) / hg);
@@ -1181,7 +1186,7 @@ static int dispatch_cut(PrefillArgs& a, const CutShape& c, int Hkv, hipStream_t 
 template <typename T, int D>
 static int dispatch_hg(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows, int64_t max_keys,
                        hipStream_t stream) {
-  switch (prefill_shape(a.R, a.group, Hkv, D, max_q_len, n_rows, max_keys)) {
+  switch (prefill_shape(a.R, a.group, Hkv, max_q_len, n_rows, max_keys)) {
     case PrefillShape::kW4Short: return dispatch_hg_w<T, D, 4, 2, 32, 3>(a, Hkv, max_q_len, n_rows, stream);
     case PrefillShape::kW4:
       // Two key halves per workgroup (8 waves, one workgroup and two waves per SIMD per
@@ -1221,6 +1226,20 @@ extern "C" int64_t ts_prefill_workspace(int R, int Hq, int Hkv, int D, int block
     return 0;
   return kCutPlanFloats + static_cast<int64_t>(c.units) * Hkv * c.hchunks * c.waves *
          (D == 128 ? cut_state_floats<128>() : cut_state_floats<64>());
+}
+
+extern "C" int ts_prefill_plan(int R, int Hq, int Hkv, int D, int block_size, int max_q_len, int64_t n_rows,
+                               int64_t max_keys, int dtype) {
+  if (R <= 0 || max_q_len <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || !is_pow2(Hq / Hkv) || !is_pow2(block_size))
+    return TS_EINVAL;
+  if ((dtype != TS_F16 && dtype != TS_BF16) || (D != 64 && D != 128)) return 0;
+  CutShape c;
+  if (cut_shape(R, Hq / Hkv, Hkv, D, ilog2(block_size), max_q_len, max_keys, &c)) return c.waves == 4 ? 5 : 4;
+  switch (prefill_shape(R, Hq / Hkv, Hkv, max_q_len, n_rows, max_keys)) {
+    case PrefillShape::kW8: return 1;
+    case PrefillShape::kW4: return 2;
+    default: return 3;
+  }
 }
 
 extern "C" int ts_prefill_varlen(const void* q, const void* k_cache, const void* v_cache,

@@ -31,6 +31,19 @@ from tinyserve_amd import _lib
 DEFAULT_TILE = (64, 32, 8)
 
 
+SHAPES = ("rows", "eight_wave", "key_split", "short_tiles", "cut_eight_wave", "cut_key_split")
+
+
+def prefill_plan(r: int, hq: int, hkv: int, d: int, block_size: int, max_q_len: int, n_rows: int, max_keys: int,
+                 dtype: torch.dtype = torch.float16) -> str:  # fmt: skip
+    """Which of ``SHAPES`` a launch of these sizes runs (``n_rows``: rows of ``q``; ``max_keys``:
+    the block table's width in keys), without launching."""
+    i = _lib.load().ts_prefill_plan(r, hq, hkv, d, block_size, max_q_len, n_rows, max_keys, _lib.DTYPES[dtype])
+    if i < 0:
+        raise ValueError(f"ts_prefill_plan: {_lib.load().ts_strerror(i).decode()}")
+    return SHAPES[i]
+
+
 @functools.lru_cache(maxsize=4096)
 def _workspace_floats(device: int, r: int, hq: int, hkv: int, d: int, block_size: int, max_q_len: int,
                       max_keys: int, dtype: torch.dtype) -> int:  # fmt: skip
