@@ -10,6 +10,8 @@ tests/helpers.py.
 
 from __future__ import annotations
 
+from dataclasses import replace
+
 import pytest
 import torch
 from hypothesis import given, settings
@@ -47,6 +49,19 @@ def check(c: PrefillCase, out: torch.Tensor) -> None:
         s, n = int(c.starts[r]), int(c.q_lens[r])
         assert torch.isfinite(out[s : s + n]).all(), f"sequence {r} read an unowned slot"
         assert_matches(out[s : s + n], want[s : s + n], c.q.dtype, f"sequence {r}")
+
+
+def widened(c: PrefillCase, tokens: int) -> PrefillCase:
+    """``c`` under a table of ``tokens`` keys (padding repeats the NaN block)."""
+    pad = c.tables[:, -1:].expand(-1, max(tokens // c.block_size - c.tables.shape[1], 0))
+    return replace(c, tables=torch.cat([c.tables, pad], dim=1).contiguous())
+
+
+def shape_of(c: PrefillCase) -> str:
+    """The workgroup shape the launch of ``c`` runs."""
+    return hip_prefill.prefill_plan(c.tables.shape[0], c.q.shape[1], c.k.shape[1], c.q.shape[2], c.block_size,
+                                    c.max_q_len, c.q.shape[0], c.tables.shape[1] * c.block_size,
+                                    c.q.dtype)  # fmt: skip
 
 
 SHAPES = [(4, 4, 8), (4, 2, 8), (4, 1, 8), (16, 8, 128), (8, 2, 64), (16, 2, 128)]
@@ -253,6 +268,25 @@ def test_long_keys_cut_over_workgroups(dtype: torch.dtype, heads: tuple[int, int
         c = prefill_case(specs, hq, hkv, d, bs, dtype, seed=bs + len(specs), gap=1)
         assert hip_prefill._workspace_floats(0, len(specs), hq, hkv, d, bs, c.max_q_len,
                                              c.tables.shape[1] * bs, dtype) > 0  # fmt: skip
+        out = torch.full_like(c.q, 7.0).to(DEVICE)
+        run(c, out=out)
+        check(c, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads", [(16, 8, 128), (32, 8, 128), (8, 2, 64), (8, 1, 128)])
+def test_short_contexts_under_wide_tables(dtype: torch.dtype, heads: tuple[int, int, int]) -> None:
+    # The table's width is the launch's bound on its keys: short contexts under a wide one run
+    # the key cut with every item whole, unpriced up to 640 keys and priced from there on (700
+    # cached tokens), in the key-split and the 8-wave shape, some sequences shorter than the
+    # longest's tiles; 60 sequences fill most of a wave's lanes.
+    cases = [[(0, 100)], [(0, 128), (0, 1), (300, 40), (0, 128)], [(0, 40)] * 3, [(0, 250), (3, 17)],
+             [(700, 20), (0, 30)]]  # fmt: skip
+    if heads[1] == 1:
+        cases = [*cases[:3], [(i, 1 + (5 * i) % 32) for i in range(60)]]
+    for specs in cases:
+        c = widened(prefill_case(specs, *heads, 16, dtype, seed=len(specs), gap=1), 16384)
+        assert shape_of(c).startswith("cut"), specs
         out = torch.full_like(c.q, 7.0).to(DEVICE)
         run(c, out=out)
         check(c, out)

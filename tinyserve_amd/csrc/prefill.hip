@@ -138,6 +138,12 @@ constexpr int kCutKeys = 64;  // keys per tile of the cut shapes
 // per part of the longest item; all three are twice as many of the shorter steps of D = 64.
 constexpr float kWholeUnit = 2.0f, kCutUnit = 4.0f, kCutMerge = 4.0f, kCutPart = 0.25f;
 
+// No share of four tiles or more is cheaper than whole items of up to this many (4 + kCutUnit +
+// kCutMerge against t + kWholeUnit steps, at D = 64 with the longer terms doubled). Such launches,
+// short contexts under wide tables, skip the pricing: 16 x 100 fresh tokens under a table of
+// 4096 13.1 -> 10.8 us (uncut 9.2), 1 x 40 9.8 -> 8.8 (6.8).
+constexpr int kCutNever = 10;
+
 struct CutItem {
   int item;   // r * n_qtiles + tile; -1: this unit has no work
   int part;   // of `parts`
@@ -163,6 +169,16 @@ __device__ __forceinline__ CutItem cut_plan(const PrefillArgs& a, int BQ) {
   const int lane = threadIdx.x & (kWave - 1);
   const int items = a.R * a.n_qtiles;
   const int t = lane < items ? cut_tiles(a, lane, BQ) : 0;
+  CutItem c;
+  c.item = lane;
+  c.part = 0;
+  const uint64_t live_items = __ballot(t > 0);
+  if (__all(t <= kCutNever)) {
+    c.parts = t > 0;
+    c.tiles = t;
+    c.unit0 = __popcll(live_items & ((uint64_t{1} << lane) - 1));
+    return c;
+  }
   const float share = __builtin_floorf(4.0f * fast_exp2(static_cast<float>(lane) * 0.1635f));
   const float inv = 1.0f / share;
   float n = 0.f, total = 0.f, tmax = 1.f, live = 0.f;
@@ -189,9 +205,7 @@ __device__ __forceinline__ CutItem cut_plan(const PrefillArgs& a, int BQ) {
   for (int o = 1; o < kWave; o *= 2) key = min(key, __shfl_xor(key, o));
   const int win = kWave - 1 - (__builtin_amdgcn_readfirstlane(key) & (kWave - 1));
   const float win_inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), win));
-  CutItem c;
-  c.item = lane;
-  c.part = c.parts = c.tiles = c.unit0 = 0;
+  c.parts = c.tiles = c.unit0 = 0;
   if (t > 0) {
     c.parts = win == kWave - 1 ? 1 : max(static_cast<int>(__builtin_ceilf(static_cast<float>(t) * win_inv - 1e-3f)), 1);
     c.tiles = (t + c.parts - 1) / c.parts;
@@ -1098,8 +1112,11 @@ static PrefillShape prefill_shape(int R, int group, int Hkv, int max_q_len, int6
 }
 
 // ---- the key cut's launches --------------------------------------------------------------
-// Its two shapes, both over 64-key tiles: up to 64 new tokens per sequence the key-split
-// one (64 queries x 2 heads, two key halves inside the workgroup), else the 8-wave one.
+// Its two shapes, both over 64-key tiles: the key-split one (64 queries x 2 heads, two key
+// halves inside the workgroup) up to 64 new tokens per sequence and where the launch would
+// run it uncut, so that a launch with nothing to cut (short contexts under a wide table) costs
+// no more than the plan and the merge's launch (1 x 500 fresh tokens under 16384 keys: 18.8 us
+// in the 8-wave shape, 14.1 in this, 13.1 uncut); else the 8-wave one.
 struct CutShape {
   int hg, waves;  // heads per workgroup; waves over the queries and heads
   int n_qtiles, hchunks, units, conc;
@@ -1118,7 +1135,8 @@ struct CutShape {
 static bool cut_shape(int R, int group, int Hkv, int D, int lbs, int max_q_len, int64_t max_keys, CutShape* c) {
   if (max_q_len > 512 || max_keys < 1024 || max_keys < 4 * static_cast<int64_t>(max_q_len)) return false;
   if ((1 << lbs) < kWave / (D / 8)) return false;  // scalar-id gather
-  c->waves = max_q_len <= 64 && group <= 4 ? 4 : 8;
+  const bool halves = prefill_shape(R, group, Hkv, max_q_len, 0, max_keys) == PrefillShape::kW4;
+  c->waves = (halves || max_q_len <= 64) && group <= 4 ? 4 : 8;
   c->hg = group < c->waves ? group : c->waves;
   c->hchunks = group / c->hg;
   const int bq = 32 * (c->waves / c->hg);
@@ -1129,7 +1147,6 @@ static bool cut_shape(int R, int group, int Hkv, int D, int lbs, int max_q_len, 
   if (items > kWave) return false;
   // What a cut can gain, in steps of the longest workgroup of the shape that runs
   // otherwise (`fill`: its workgroups per CU).
-  const bool halves = prefill_shape(R, group, Hkv, max_q_len, 0, max_keys) == PrefillShape::kW4;
   if (!halves && max_q_len > 128) return false;
   const int hg = halves ? std::min(group, 4) : std::min(group, 8);
   const int oq = 32 * ((halves ? 4 : 8) / hg);

@@ -82,7 +82,11 @@ def paged_prefill_attention(
         q: ``[T, Hq, D]`` queries after RoPE; rows no prompt claims are not read.
         k_cache, v_cache: one layer of the cache, ``[num_slots, Hkv, D]``, already
             holding this step's keys and values.
-        block_tables: int32 ``[R, max_blocks]``.
+        block_tables: int32 ``[R, max_blocks]``. Its width is the launch's only bound on the
+            contexts (lengths are on the device): wide against ``max_q_len`` it plans for long
+            cached keys, a second kernel and a workspace of up to 69 MB included. Pass it no
+            wider than the longest context needs (``block_tables[:, :n]``, a view); under a table
+            of 4096 tokens 16 prompts of 100 take 10.8 us in place of 8.0, one of 40 8.8 for 5.6.
         q_starts, q_lens, context_lens: int32 ``[R]``.
         max_q_len: host-side maximum of ``q_lens``; it sizes the grid, so nothing is read
             back from the device.
