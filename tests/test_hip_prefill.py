@@ -292,6 +292,16 @@ def test_short_contexts_under_wide_tables(dtype: torch.dtype, heads: tuple[int, 
         check(c, out)
 
 
+@pytest.mark.parametrize("specs", [[(3000, 20)], [(3000, 100), (0, 9)], [(700, 60)], [(0, 500)]])
+def test_scores_far_below_zero(specs: list[tuple[int, int]]) -> None:
+    # Every score -2^110 (exact, so every weight is equal): key parts and halves that start
+    # past the first key must take their own maximum, whatever it is.
+    c = prefill_case(specs, 16, 8, 128, 16, torch.bfloat16, seed=len(specs), sentinel=False)
+    c = replace(c, q=torch.full_like(c.q, 2.0**50), k=torch.full_like(c.k, -(2.0**53)))
+    assert "key_split" in shape_of(c) or "cut" in shape_of(c)
+    check(c, run(c))
+
+
 def test_cut_launch_replays_in_a_graph() -> None:
     c = on_gpu(prefill_case([(2500, 90), (100, 20)], 16, 8, 128, 16, torch.float16, seed=5))
     want = paged_prefill_attention(*c.args())

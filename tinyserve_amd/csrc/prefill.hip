@@ -123,6 +123,9 @@ struct PrefillArgs {
 };
 
 constexpr int kWin = 512;   // block ids held in LDS
+// Before any score: at or below every finite one, so a part of very low scores (bf16 reaches
+// -1e34) still starts from its own maximum.
+constexpr float kLowest = -3.402823466e38f;
 constexpr int kCutKeys = 64;  // keys per tile of the cut shapes
 
 // ---- key cut -----------------------------------------------------------------------------
@@ -467,7 +470,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
   f32x16 oacc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x16{};
-  float m_run = -1.0e30f;  // running max of scale*log2e*score; finite, so 2^(m_run - x) is 0
+  float m_run = kLowest;  // running max of scale*log2e*score; finite, so 2^(m_run - x) is 0
   float l_run = 0.f;       // this lane half's share of the softmax denominator
 
   // ---- the gather: one tile of K and V into a ring stage --------------------------------
@@ -947,7 +950,7 @@ __global__ __launch_bounds__(PG * D / 32 * kWave) void prefill_merge_kernel(cons
   const int64_t stride = static_cast<int64_t>(n_hc) * GW * cut_state_floats<D>();  // one unit
   const float* st = a.ws + unit0 * stride + (static_cast<int64_t>(hcx) * GW + wl) * cut_state_floats<D>();
   const float* ml = st + D / 2 * kWave + lane;
-  float m = -1.0e30f;
+  float m = kLowest;
 #pragma unroll 8
   for (int i = pg; i < parts; i += PG) m = fmaxf(m, ml[i * stride]);
   float l = 0.f;
