@@ -211,12 +211,18 @@ def test_compiled_binding_passes_the_declared_arguments(lib: ctypes.CDLL) -> Non
 
 
 def test_policy_splits_of_four_head_tiles(lib: ctypes.CDLL) -> None:
-    # Half the chip's SIMDs exactly (16 sequences of 8 eight-wave workgroups) is split into
-    # partials at four heads of 128 elements; more is one launch, as at two heads or 64.
-    policy = hip_attention.policy_splits
-    assert policy(16, 32, 8, 128, 16, 256) > 1
-    assert policy(17, 32, 8, 128, 16, 256) == 1 and policy(48, 32, 8, 128, 16, 256) == 1
-    assert policy(16, 16, 8, 128, 16, 256) == 1
+    # The ranges of four waves that one round holds, 2048 // (4 x tiles): four up to 16
+    # sequences of 8 tiles, three up to 21, no more than one launch's eight waves from 22 on;
+    # over tables of 850 tokens / (ranges - 2) at least. Other tiles keep their rule.
+    def policy(b: int, width: int, hq: int = 32, hkv: int = 8, d: int = 128) -> int:
+        return hip_attention.policy_splits(b, hq, hkv, d, 16, width)
+
+    assert [policy(b, 256) for b in (1, 8, 15, 16, 17, 21, 22, 48, 200)] == [16, 8, 4, 4, 3, 3, 1, 1, 1]
+    assert policy(16, 26) == 1 and policy(16, 27) == 4  # 416, 432 tokens
+    assert policy(17, 53) == 1 and policy(17, 54) == 3  # 848, 864
+    assert policy(8, 256, hq=64) == 4 and policy(11, 256, hq=64) == 1 and policy(34, 256, hq=16, hkv=4) == 3
+    assert policy(17, 256, d=256) == 3 and policy(17, 256, d=64) == 1
+    assert policy(16, 256, hq=16) == 1
 
 
 def test_policy_runs_short_tables_as_one_launch(lib: ctypes.CDLL) -> None:

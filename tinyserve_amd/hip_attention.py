@@ -74,6 +74,17 @@ IN_GROUP_MIN_WAVES = 1024
 # against 18-19 (two launches and three allocations of host time).
 ONE_LAUNCH_TOKEN_HEADS = 512
 
+# Tiles of four query heads of 128 elements or more run two waves per SIMD; the policy splits
+# them into the ranges of four waves that one round of the chip holds, 2048 waves // (4 x tiles),
+# where that is more waves per tile than one launch's eight, over tables of at least this many
+# tokens / (ranges - 2): what a range saves must pay the partials and the second launch.
+# Measured (one launch against ranges, us, 32 q / 8 kv heads fp16, equal and U[1, n] lengths):
+# 16 sequences in 4 (half the chip) 300 tokens 13.2 against 14.1, 12.9 / 13.8; 512 15.9 / 15.3, 15.1
+# / 14.2; 4096 71 / 49, 67 / 43; 17 in 3 512 tokens 16.1 / 17.4, 15.2 / 15.6; 1024 24.3 / 23.8, 23.7 /
+# 19.7; 4096 75 / 58, 68 / 43; 21 in 3 4096 83 / 77, 68 / 43; 22, which holds only two, in 3 4096
+# 84 / 101, 68 / 78. The same at 16 / 4 and 64 / 8 heads, fp32 and 256 elements.
+WIDE_RANGE_TOKENS = 850
+
 # Reference constants, kept for ``num_splits_for(..., target=..., no_split=...)`` callers
 # that want the T4 policy exactly.
 T4_TARGET_PROGRAMS = 1024
@@ -187,17 +198,19 @@ def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int
     sequence over their waves. A smaller grid gets enough split ranges for about twice
     the chip (at most ``MAX_SPLITS`` and the table width), as fp32 partials and the
     combine, unless its tables are so short (``ONE_LAUNCH_TOKEN_HEADS``) that one launch is
-    faster. Sizes only (``device`` sets the CU count): a graph-captured launch keeps its
-    grid."""
+    faster. Tiles of four heads of 128 elements or more follow ``WIDE_RANGE_TOKENS`` instead.
+    Sizes only (``device`` sets the CU count): a graph-captured launch keeps its grid."""
     splits = num_splits_for(batch, num_kv_heads, max_blocks)
     simds = _one_split_waves(device, batch, num_q_heads, num_kv_heads, head_dim, block_size,
                              max_blocks, dtype)  # fmt: skip
     heads = min(num_q_heads // num_kv_heads, 4)  # per wave
     if head_dim <= 128 and max_blocks * block_size * heads <= ONE_LAUNCH_TOKEN_HEADS:
         return 1
-    # Four-head tiles of 128 elements: just half the chip is not enough (32 q / 8 kv heads bf16
-    # 16 x 4096: one launch 78 us, partials 50; 16 x U[100, 5000] 91 and 56).
-    if simds >= IN_GROUP_MIN_WAVES // 2 + (heads == 4 and head_dim >= 128):
+    if heads == 4 and head_dim >= 128:
+        tiles = batch * num_q_heads // heads
+        ranges = min(IN_GROUP_MIN_WAVES // (2 * tiles), MAX_SPLITS, max_blocks)
+        return ranges if max_blocks * block_size * (ranges - 2) >= WIDE_RANGE_TOKENS else 1
+    if simds >= IN_GROUP_MIN_WAVES // 2:
         return 1 if splits <= IN_GROUP_SPLITS else splits
     return max(splits, min(-(-2 * IN_GROUP_MIN_WAVES // max(simds, 1)), MAX_SPLITS, max_blocks))
 
