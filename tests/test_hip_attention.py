@@ -617,13 +617,29 @@ def test_small_grid_policy_replays_in_a_graph(lens: list[int]) -> None:
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("batch,splits", [(40, 1), (40, 4), (40, 12), (16, None), (16, 1), (3, None), (70, 1)])
 def test_four_head_tiles_of_128_elements(batch: int, splits: int | None, dtype: torch.dtype) -> None:
-    # Two waves per SIMD: length pairs of eight waves (40), the in-group split ranges of eight
-    # waves and, where their states do not fit the LDS, of four (4 and 12 splits), plain
-    # workgroups of eight, the policy's partials, and several workgroups per CU (70).
+    # Two waves per SIMD: length pairs of eight waves (40), explicit counts as partials (40 x 4
+    # and 12: the grid is under the chip), plain workgroups of eight, the policy's partials,
+    # and several workgroups per CU (70).
     c = decode_case([1 + (389 * i) % 1100 for i in range(batch)], 32, 8, dtype=dtype, seed=batch)
     g = on_gpu(c)
     out = ha.launch_paged_decode_split(*g.args(), c.scale, c.block_size, num_splits=splits)
     assert_matches(out, oracle32(c), dtype, f"{batch} sequences, {splits} splits")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,splits", [(40, 4), (40, 7), (40, 8), (40, 11), (20, 16), (20, 27)])
+def test_in_group_splits_of_four_head_tiles(batch: int, splits: int, dtype: torch.dtype) -> None:
+    # Split ranges inside the workgroups: length pairs of eight waves up to 7 ranges, of four
+    # from 8 to 11, where the states of eight pass 64 KiB, and refused from 12 on; plain
+    # workgroups of eight up to 23 and of four up to 27.
+    c = decode_case([1 + (389 * i) % 1100 for i in range(batch)], 32, 8, dtype=dtype, seed=batch + splits)
+    g = on_gpu(c)
+    plan = ha.decode_plan(batch, 32, 8, 128, c.block_size, g.block_tables.shape[1], 1, dtype=dtype)
+    assert (plan["budget"], plan["waves_per_group"], plan["by_length"]) == ("light_wide", 8, batch == 40)
+    assert_matches(in_group_split(g, splits), oracle32(c), dtype, f"{batch} sequences, {splits} splits")
+    with pytest.raises(ValueError, match="unsupported"):
+        in_group_split(g, 12 if batch == 40 else 28)
 
 
 @pytest.mark.gpu
