@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import sysconfig
 from pathlib import Path
 
 import pytest
@@ -194,7 +195,7 @@ def test_compiled_binding_passes_the_declared_arguments(lib: ctypes.CDLL) -> Non
     # status for the same arguments.
     from tinyserve_amd import _fastcall
 
-    kinds = {_lib._vp: "P", _lib._i: "I", _lib._i64: "L", _lib._f: "F", ctypes.c_double: "F"}
+    kinds = _lib._KINDS
     source = (Path(_lib.__file__).parent / "csrc" / "fastcall.c").read_text()
     entries = re.findall(r"^ENTRY\((\w+), (\d+),\n(.*?)\)$", source, re.M | re.S)
     assert {name for name, _, _ in entries} == set(_lib._fns) & {n for n in dir(_fastcall) if n.startswith("ts_")}
@@ -208,6 +209,27 @@ def test_compiled_binding_passes_the_declared_arguments(lib: ctypes.CDLL) -> Non
         assert getattr(_fastcall, name)(*zeros) == getattr(lib, name)(*zeros)
     with pytest.raises(TypeError):
         _fastcall.ts_silu_mul("x", 0, 0, 0, 0, 0, 0, 0)
+    with pytest.raises(TypeError):  # None is a pointer's, as in ctypes; the first fault is reported
+        _fastcall.ts_silu_mul(None, None, None, "x", 0, 0, 0, None)
+    # Another argument list than the module's is not bound.
+    want = "".join(kinds[t] for t in _lib.SIGNATURES["ts_silu_mul"][1])
+    at = ctypes.cast(lib.ts_silu_mul, ctypes.c_void_p).value
+    for other in ("", want[:-1], want + "P", want.replace("L", "I")):
+        assert not _fastcall.bind("ts_silu_mul", at, other)
+    assert _fastcall.bind("ts_silu_mul", at, want) and not _fastcall.bind("ts_version", at, "")
+
+
+def test_builds_without_the_compiled_binding(tmp_path: Path, monkeypatch) -> None:  # noqa: ANN001
+    # No headers: the build goes on, and says so; the name carries the interpreter's tag.
+    from tinyserve_amd import build
+
+    monkeypatch.setattr(build, "PKG", tmp_path)
+    out = build._build_fastcall(False)
+    assert out is not None and out.name == "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX")
+    out.unlink()
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build._build_fastcall(False) is None
+    assert not list(tmp_path.glob("_fastcall*.so"))
 
 
 def test_policy_splits_of_four_head_tiles(lib: ctypes.CDLL) -> None:

@@ -109,15 +109,21 @@ def load() -> ctypes.CDLL:
 _fns: dict[str, object] = {}
 
 
+# Argument kinds as fastcall.c writes them.
+_KINDS = {_vp: "P", _i: "I", _i64: "L", _f: "F", ctypes.c_double: "F"}
+
+
 def _bind_fast(lib: ctypes.CDLL) -> None:
-    """Fill ``_fns`` with the compiled binding's functions, pointed at ``lib``'s entry points
-    (none without the built module: every call then goes through ctypes)."""
+    """Fill ``_fns`` with the compiled binding's functions, pointed at ``lib``'s entry points.
+    Without the built module, or where it was built from other argument lists, calls go
+    through ctypes."""
     try:
         from tinyserve_amd import _fastcall
     except ImportError:
         return
     for name in EXPORTS:
-        if _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value):
+        kinds = "".join(_KINDS.get(t, "?") for t in SIGNATURES[name][1])
+        if _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value, kinds):
             _fns[name] = getattr(_fastcall, name)
 
 

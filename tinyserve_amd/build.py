@@ -81,15 +81,19 @@ def build(verbose: bool = False) -> Path:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
+    for old in PKG.glob("_fastcall*.so"):  # built from the sources of the library that goes
+        old.unlink()
     tmp.replace(out)  # atomic: a process that already mapped the old file keeps it
     _build_fastcall(verbose)
     return out
 
 
-def _build_fastcall(verbose: bool) -> None:
-    """The compiled Python binding of the launch entry points (host code only)."""
+def _build_fastcall(verbose: bool) -> Path | None:
+    """The compiled Python binding of the launch entry points (host code only), named for the
+    interpreter it is built for. Without a C compiler or Python's headers there is none, and
+    calls go through ctypes."""
     cc = shutil.which("gcc") or shutil.which("cc") or hipcc()
-    out = PKG / "_fastcall.so"
+    out = PKG / f"_fastcall{sysconfig.get_config_var('EXT_SUFFIX')}"
     tmp = out.with_suffix(".so.tmp")
     cmd = [cc, "-O2", "-fPIC", "-shared", f"-I{sysconfig.get_paths()['include']}", str(CSRC / "fastcall.c"),
            "-o", str(tmp)]  # fmt: skip
@@ -97,8 +101,10 @@ def _build_fastcall(verbose: bool) -> None:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
-        raise RuntimeError(f"fastcall.c failed:\n{proc.stderr}")
+        print(f"fastcall.c failed; launches go through ctypes:\n{proc.stderr}", file=sys.stderr)
+        return None
     tmp.replace(out)
+    return out
 
 
 if __name__ == "__main__":

@@ -3,8 +3,9 @@
  * launch took ctypes 2.4 us, this 0.5 us. Same functions, same arguments, same status; the
  * binding passes the addresses it looked up (bind), so there is one copy of the library.
  *
- * Integers convert as ctypes converts them (a Python int, or None for a null pointer, cut to
- * the parameter's width); the interpreter lock is released for the call.
+ * Integers convert as ctypes converts them (a Python int, cut to the parameter's width; None
+ * for a null pointer only), floats as PyFloat_AsDouble takes them; the interpreter lock is
+ * released for the call.
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -12,10 +13,6 @@
 #include <string.h>
 
 #include "../../include/tinyserve_amd.h"
-
-static int64_t as_int(PyObject* o) {
-  return o == Py_None ? 0 : (int64_t)PyLong_AsUnsignedLongLongMask(o);
-}
 
 #define P(i) (void*)(uintptr_t)v[i].n
 #define I(i) (int)v[i].n
@@ -29,23 +26,37 @@ typedef union {
 
 enum { kMaxArgs = 40 };
 
-/* `kinds`: the argument list's macro names, whose letters say which are floating. */
+/* The next argument's kind (P, I, L or F; 0 at the end) of a list of macro names. */
+static char next_kind(const char** kinds) {
+  for (; **kinds; ++*kinds)
+    if (strchr("PILF", **kinds)) return *(*kinds)++;
+  return 0;
+}
+
+/* `kinds`: the argument list's macro names. */
 static int convert(const char* name, const char* kinds, int want, PyObject* const* a, Py_ssize_t n, Arg* v) {
   if (n != want) {
     PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %zd", name, want, n);
     return -1;
   }
-  const char* k = kinds;
   for (int i = 0; i < want; ++i) {
-    while (*k != 'P' && *k != 'I' && *k != 'L' && *k != 'F') ++k;
-    if (*k++ == 'F') v[i].f = PyFloat_AsDouble(a[i]);
-    else v[i].n = as_int(a[i]);
+    const char k = next_kind(&kinds);
+    if (k == 'F') {
+      v[i].f = PyFloat_AsDouble(a[i]);
+      if (v[i].f == -1.0 && PyErr_Occurred()) return -1;
+    } else if (k == 'P' && a[i] == Py_None) {
+      v[i].n = 0;
+    } else {
+      v[i].n = (int64_t)PyLong_AsUnsignedLongLongMask(a[i]);
+      if (v[i].n == -1 && PyErr_Occurred()) return -1;
+    }
   }
-  return PyErr_Occurred() ? -1 : 0;
+  return 0;
 }
 
 #define ENTRY(NAME, N, ...)                                                          \
   static __typeof__(&NAME) p_##NAME;                                                 \
+  static const char k_##NAME[] = #__VA_ARGS__;                                       \
   static PyObject* call_##NAME(PyObject* self, PyObject* const* a, Py_ssize_t n) {   \
     Arg v[kMaxArgs];                                                                 \
     int rc;                                                                          \
@@ -54,7 +65,7 @@ static int convert(const char* name, const char* kinds, int want, PyObject* cons
       PyErr_SetString(PyExc_RuntimeError, #NAME " is not bound");                    \
       return NULL;                                                                   \
     }                                                                                \
-    if (convert(#NAME, #__VA_ARGS__, N, a, n, v)) return NULL;                       \
+    if (convert(#NAME, k_##NAME, N, a, n, v)) return NULL;                           \
     Py_BEGIN_ALLOW_THREADS                                                           \
     rc = p_##NAME(__VA_ARGS__);                                                      \
     Py_END_ALLOW_THREADS                                                             \
@@ -101,14 +112,23 @@ ENTRY(ts_add_rms_norm, 15,
   X(ts_rows_gemm)                                                                   \
   X(ts_add_rms_norm)
 
-/* bind(name, address): where the library has the entry point. False for a name not here. */
+/* Whether an argument list's letters are `want`, letter for letter. */
+static int same_kinds(const char* kinds, const char* want) {
+  char k;
+  while ((k = next_kind(&kinds)) && k == *want) ++want;
+  return k == 0 && *want == 0;
+}
+
+/* bind(name, address, kinds): where the library has the entry point, and the kinds of its
+ * arguments ("PPIL..."). False, unbound, for a name that is not here or has others. */
 static PyObject* bind(PyObject* self, PyObject* args) {
-  const char* name;
+  const char *name, *kinds;
   unsigned long long at;
   (void)self;
-  if (!PyArg_ParseTuple(args, "sK", &name, &at)) return NULL;
+  if (!PyArg_ParseTuple(args, "sKs", &name, &at, &kinds)) return NULL;
 #define BIND(NAME)                                          \
   if (strcmp(name, #NAME) == 0) {                           \
+    if (!same_kinds(k_##NAME, kinds)) Py_RETURN_FALSE;      \
     p_##NAME = (__typeof__(&NAME))(uintptr_t)at;            \
     Py_RETURN_TRUE;                                         \
   }
