@@ -218,3 +218,17 @@ def test_rope_tables_of_many_positions(t: int) -> None:
     for at in (0, t // 2, t - 5):
         c, s = rope_cos_sin(128, 1.0e6, pos[at : at + 5])
         assert torch.equal(cos[at : at + 5], c) and torch.equal(sin[at : at + 5], s)
+
+
+def test_rope_tables_up_to_the_last_position_count() -> None:
+    # 2^31 - 2 positions, the counts' end: the last thread's four positions pass INT_MAX.
+    t = 2**31 - 2
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 48 GiB")
+    pos = torch.arange(t, device=DEVICE)
+    cos, sin = rope_cos_sin(2, 1.0e6, pos)
+    for at in (0, t // 2, t - 5):
+        c, s = rope_cos_sin(2, 1.0e6, pos[at : at + 5])
+        assert torch.equal(cos[at : at + 5], c) and torch.equal(sin[at : at + 5], s)
+    del pos, cos, sin
+    torch.cuda.empty_cache()

@@ -407,7 +407,8 @@ __global__ __launch_bounds__(256) void rope_cos_sin_kernel(const int64_t* __rest
                                                            float* __restrict__ sin_out, int64_t stride) {
   const int half = D / 2;
   const int64_t u = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int t0 = static_cast<int>(u / half) * PPT, i = static_cast<int>(u % half);
+  const int64_t t0 = u / half * PPT;  // the last thread's may pass INT_MAX
+  const int i = static_cast<int>(u % half);
   if (t0 >= T) return;
   int64_t p[PPT];
 #pragma unroll
@@ -440,11 +441,11 @@ extern "C" int ts_rope_cos_sin(const int64_t* positions, int T, int D, double th
   // Two positions per thread from one wave per SIMD of such threads on, four from two.
   const int64_t lanes = 4 * 64 * static_cast<int64_t>(compute_units());
   if (n >= 8 * lanes) {
-    const int64_t n4 = static_cast<int64_t>((T + 3) / 4) * (D / 2);
+    const int64_t n4 = (static_cast<int64_t>(T) + 3) / 4 * (D / 2);
     hipLaunchKernelGGL(rope_cos_sin_kernel<4>, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,
                        positions, T, D, theta, cos_out, sin_out, stride);
   } else if (n >= 2 * lanes) {
-    const int64_t n2 = static_cast<int64_t>((T + 1) / 2) * (D / 2);
+    const int64_t n2 = (static_cast<int64_t>(T) + 1) / 2 * (D / 2);
     hipLaunchKernelGGL(rope_cos_sin_kernel<2>, dim3(static_cast<unsigned>((n2 + 255) / 256)), dim3(256), 0, st,
                        positions, T, D, theta, cos_out, sin_out, stride);
   } else {
