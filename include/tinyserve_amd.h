@@ -219,8 +219,8 @@ int ts_add_rms_norm_rows(void* x, const void* y, const void* w, void* out, int T
 
 /*
  * act[t] = silu(gate_up[t][:N]) * gate_up[t][N:2N], each rounded to the type (reference
- * src/tinyserve/model.py:176-178). Rows 16-byte aligned, N a multiple of 16 bytes; others
- * return TS_EUNSUPPORTED.
+ * src/tinyserve/model.py:176-178). Rows 16-byte aligned, N a multiple of 16 bytes, at
+ * most 2^32 - 1 vectors of 16 bytes; others return TS_EUNSUPPORTED.
  */
 int ts_silu_mul(const void* gate_up, void* act, int T, int N, int64_t g_stride,
                 int64_t a_stride, int dtype, void* stream);

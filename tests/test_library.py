@@ -84,6 +84,11 @@ def test_c_abi_rejects_bad_sizes_before_any_launch(lib: ctypes.CDLL) -> None:
     assert lib.ts_rows_gemm(p, 0, 32, p, 64, p, 64, null, 0, 4, 64, 64, 0, 1, null) == -1
     assert lib.ts_rows_gemm(p, 1, 0, p, 48, p, 64, null, 0, 4, 64, 48, 0, 1, null) == -1
     assert lib.ts_rows_gemm(p, 0, 64, p, 64, p, 64, null, 0, 0, 64, 64, 0, 1, null) == 0  # no rows
+    # the fused SiLU refuses more vectors than a launch has threads (its caller takes another
+    # path), rows that are not whole 16-byte vectors, and short strides
+    assert lib.ts_silu_mul(p, p, 2**31 - 1, 64, 128, 64, 1, null) == -2
+    assert lib.ts_silu_mul(p, p, 4, 60, 120, 60, 1, null) == -2
+    assert lib.ts_silu_mul(p, p, 4, 64, 64, 64, 1, null) == -1
     # fp32 has no MFMA projection kernel
     assert lib.ts_rows_gemm(p, 0, 64, p, 64, p, 64, null, 0, 4, 64, 64, 0, 0, null) == -2
     assert lib.ts_add_rms_norm(p, 64, null, 2, p, p, 64, p, 0, 64, 4, 64, 1e-6, 1, null) == -1  # ks, no partials

@@ -227,6 +227,7 @@ static int launch_silu_mul(const void* gu, void* act, int rows, int N, int64_t g
       (reinterpret_cast<uintptr_t>(gu) | reinterpret_cast<uintptr_t>(act)) % 16)
     return TS_EUNSUPPORTED;
   const int64_t n = static_cast<int64_t>(rows) * (N / VEC);
+  if (n >> 32) return TS_EUNSUPPORTED;  // past the threads a launch may have
   hipLaunchKernelGGL(silu_mul_kernel<T>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st,
                      static_cast<const T*>(gu), static_cast<T*>(act), rows, N / VEC, N, gs, as);
   return launch_status();
