@@ -189,26 +189,32 @@ def test_baseline_config_3_against_the_batched_path(dtype: torch.dtype) -> None:
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_both_workgroup_shapes(dtype: torch.dtype) -> None:
-    # The library picks the workgroup shape from the 8-wave grid (wg8 workgroups of 128
-    # queries x 2 heads) at Qwen3 shapes on 256 CUs: 3 prompts of up to 2048 tokens make
-    # 256 (under 1.5 per CU: 4 waves, 64-key tiles, two per CU); 4 prompts make 512 and 16
-    # prompts of up to 512 tokens 512 (4 waves, 32-key tiles, three per CU); 24 prompts
-    # of up to 1408 tokens make 2112, over 8 per CU with a mean above 1280 new tokens
-    # (8 waves, 64-key tiles, many query tiles per sequence).
-    for lens in ([2048, 1999, 1100, 700], [2048, 1500, 64], [512] * 15 + [77],
-                 [1300 + (37 * i) % 109 for i in range(23)] + [1408]):  # fmt: skip
+    # The library picks the workgroup shape from the grids and the walk, at Qwen3 shapes on 256
+    # CUs: one prompt of 2048 tokens makes one round of the key-split shape; 3 and 4 prompts
+    # of up to 2048 and 16 of up to 512 make up to 8 8-wave workgroups per CU (4 waves, 32-key
+    # tiles, three per CU); 24 prompts of up to 1408 tokens make 2112, over 8 per CU with a mean
+    # above 1280 new tokens (8 waves, 64-key tiles, many query tiles per sequence).
+    for lens, shape in (([2048], "key_split"), ([2048, 1999, 1100, 700], "short_tiles"),
+                        ([2048, 1500, 64], "short_tiles"), ([512] * 15 + [77], "short_tiles"),
+                        ([1300 + (37 * i) % 109 for i in range(23)] + [1408], "eight_wave")):  # fmt: skip
         c = prefill_case([(0, n) for n in lens], 16, 8, 128, 16, dtype, seed=len(lens))
+        assert shape_of(c) == shape, lens
         check(c, run(c))
 
 
 @pytest.mark.parametrize("block_size", [1, 2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("shape", [(16, 8, 128), (8, 2, 64)])
 def test_every_gather_path_on_every_workgroup_shape(block_size: int, shape: tuple[int, int, int]) -> None:
-    # Each launch below runs one of the three workgroup shapes (one prompt: 4 waves,
-    # 64-key tiles; 16 prompts of 512: 4 waves, 32-key tiles; 4 chunks of 128 new tokens:
-    # 8 waves), with prefix hits so that tiles start mid-block, at every block size.
-    for specs in ([(70, 300)], [(33, 512)] * 15 + [(5, 77)], [(100 + 300 * i, 128) for i in range(4)]):
+    # Each launch below runs one of the three workgroup shapes (one prompt: two key halves, or
+    # 4 waves over 64-key tiles below the halves' block size; 16 prompts of 512: 4 waves,
+    # 32-key tiles; 4 chunks of 128 new tokens: 8 waves), with prefix hits so that tiles start
+    # mid-block, at every block size; the last cuts its keys where the block size allows.
+    cut = "cut_eight_wave" if block_size * shape[2] >= 512 else "eight_wave"
+    for specs, want in (([(70, 300)], "key_split"), ([(33, 512)] * 15 + [(5, 77)], "short_tiles"),
+                        ([(100 + 200 * i, 128) for i in range(4)], "eight_wave"),
+                        ([(1000 + 300 * i, 128) for i in range(4)], cut)):  # fmt: skip
         c = prefill_case(specs, *shape, block_size, torch.float16, seed=block_size)
+        assert shape_of(c) == want, specs
         check(c, run(c))
 
 
@@ -216,17 +222,39 @@ def test_every_gather_path_on_every_workgroup_shape(block_size: int, shape: tupl
 @pytest.mark.parametrize("heads", [(16, 8, 128), (32, 8, 128), (8, 2, 64)])
 def test_key_split_workgroups(dtype: torch.dtype, heads: tuple[int, int, int]) -> None:
     # One or two prompts run workgroups whose waves split the key tiles in two halves
-    # and merge at the end: one key tile (the upper half empty), odd and even tile
+    # and merge at the end: one key tile (the upper half empty) and a few, under tables of 512
+    # keys (under tight ones such prompts run the 32-key shape), odd and even tile
     # counts, a query block whose keys end before the upper half, prefix hits (the
     # halves split the cached keys too; chunks of at most 64 new tokens in small launches
-    # run this shape as well), and block sizes below the scalar-id gather's (the unsplit
-    # 4-wave kernel).
-    for specs, bs in (([(0, 1)], 16), ([(0, 64)], 16), ([(0, 65)], 16), ([(0, 200)], 16),
-                      ([(0, 1000)], 32), ([(300, 37)], 16), ([(100, 2048)], 16),
-                      ([(1024, 64)] * 4, 16), ([(8000, 50)], 16),
-                      ([(0, 700), (9, 1300)], 64), ([(0, 500)], 2), ([(33, 400)], 1)):  # fmt: skip
-        c = prefill_case(specs, *heads, bs, dtype, seed=bs + len(specs))
+    # run this shape as well, or the cut of longer keys), and block sizes below the scalar-id
+    # gather's (the unsplit 4-wave kernel).
+    for specs, bs, tokens in (([(0, 1)], 16, 512), ([(0, 64)], 16, 512), ([(0, 60), (130, 1)], 16, 512),
+                              ([(0, 200)], 16, 512), ([(0, 1000)], 32, 0), ([(300, 37)], 16, 0),
+                              ([(100, 2048)], 16, 0), ([(1024, 64)] * 4, 16, 0), ([(8000, 50)], 16, 0),
+                              ([(0, 500), (9, 700)], 64, 0), ([(0, 500)], 2, 0), ([(33, 400)], 1, 0),
+                              ([(0, 1)], 16, 0), ([(0, 64)], 16, 0), ([(0, 65)], 16, 0), ([(0, 200)], 16, 0),
+                              ([(0, 700), (9, 1300)], 64, 0)):  # fmt: skip
+        c = widened(prefill_case(specs, *heads, bs, dtype, seed=bs + len(specs)), tokens)
+        if tokens or max(n for _, n in specs) not in (1, 64, 65, 200, 1300):
+            assert shape_of(c) == ("cut_key_split" if specs[0][0] == 8000 else "key_split"), specs
         check(c, run(c))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads", [(16, 8, 128), (8, 2, 64)])
+def test_output_rows_off_16_bytes(dtype: torch.dtype, heads: tuple[int, int, int]) -> None:
+    # Output strides that are not whole 16-byte vectors: every shape stores its lanes' pieces of
+    # 8 bytes directly, whole and cut items alike.
+    for specs, want in (([(0, 70), (9, 3)], "short_tiles"), ([(0, 300)], "key_split"),
+                        ([(300, 100), (5, 33)], "eight_wave"), ([(5000, 40), (3, 9)], "cut_key_split"),
+                        ([(3000, 100), (0, 7)], "cut_eight_wave")):  # fmt: skip
+        c = prefill_case(specs, *heads, 16, dtype, seed=len(want))
+        assert shape_of(c) == want, specs
+        wide = torch.full((*c.q.shape[:2], heads[2] + 4), 7.0, dtype=dtype, device=DEVICE)
+        out = wide[:, :, : heads[2]]
+        run(c, out=out)
+        check(c, out)
+        assert bool((wide[:, :, heads[2] :] == 7.0).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
