@@ -33,14 +33,14 @@ static char next_kind(const char** kinds) {
   return 0;
 }
 
-/* `kinds`: the argument list's macro names. */
+/* `kinds`: each argument's. */
 static int convert(const char* name, const char* kinds, int want, PyObject* const* a, Py_ssize_t n, Arg* v) {
   if (n != want) {
     PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %zd", name, want, n);
     return -1;
   }
   for (int i = 0; i < want; ++i) {
-    const char k = next_kind(&kinds);
+    const char k = kinds[i];
     if (k == 'F') {
       v[i].f = PyFloat_AsDouble(a[i]);
       if (v[i].f == -1.0 && PyErr_Occurred()) return -1;
@@ -56,7 +56,8 @@ static int convert(const char* name, const char* kinds, int want, PyObject* cons
 
 #define ENTRY(NAME, N, ...)                                                          \
   static __typeof__(&NAME) p_##NAME;                                                 \
-  static const char k_##NAME[] = #__VA_ARGS__;                                       \
+  static const char list_##NAME[] = #__VA_ARGS__;                                    \
+  static char k_##NAME[kMaxArgs]; /* its kinds, from bind */                         \
   static PyObject* call_##NAME(PyObject* self, PyObject* const* a, Py_ssize_t n) {   \
     Arg v[kMaxArgs];                                                                 \
     int rc;                                                                          \
@@ -128,7 +129,8 @@ static PyObject* bind(PyObject* self, PyObject* args) {
   if (!PyArg_ParseTuple(args, "sKs", &name, &at, &kinds)) return NULL;
 #define BIND(NAME)                                          \
   if (strcmp(name, #NAME) == 0) {                           \
-    if (!same_kinds(k_##NAME, kinds)) Py_RETURN_FALSE;      \
+    if (!same_kinds(list_##NAME, kinds)) Py_RETURN_FALSE;   \
+    strcpy(k_##NAME, kinds);                                \
     p_##NAME = (__typeof__(&NAME))(uintptr_t)at;            \
     Py_RETURN_TRUE;                                         \
   }
