@@ -258,6 +258,10 @@ def test_policy_runs_short_tables_as_one_launch(lib: ctypes.CDLL) -> None:
     for hq, line in ((8, 32), (16, 16), (32, 8), (64, 8)):
         assert hip_attention.policy_splits(4, hq, 8, 128, 16, line) == 1
         assert hip_attention.policy_splits(4, hq, 8, 128, 16, line + 1) > 1
+    # 32-bit rows of 128 elements: 160 KB of K per kv head.
+    assert hip_attention.policy_splits(4, 8, 8, 128, 16, 20, torch.float32) == 1
+    assert hip_attention.policy_splits(4, 8, 8, 128, 16, 21, torch.float32) > 1
+    assert hip_attention.policy_splits(4, 8, 8, 64, 16, 32, torch.float32) == 1
 
 
 @pytest.mark.parametrize(("heads", "specs", "want"), [

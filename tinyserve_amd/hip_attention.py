@@ -71,8 +71,11 @@ IN_GROUP_MIN_WAVES = 1024
 # policy's partials, us): 16 q / 8 kv heads fp16 208 tokens 6.9 against 7.6-8.4, 256 tokens
 # 6.9 against 7.8-8.4, fp32 256 tokens 7.7 against 8.2-8.6; 32 / 8 heads (four per wave) 128
 # tokens 7.8 against 9.1-10.1 but 208 tokens 10.8 against 9.2-11.0; called eagerly, 8.5-9.2
-# against 18-19 (two launches and three allocations of host time).
+# against 18-19 (two launches and three allocations of host time). The table's K per kv head is
+# bounded too: 32-bit rows of 128 elements at one head per wave are 7.5-8.2 us at 256 tokens
+# either way, 8.0-8.2 against 7.5-8.1 at 384 and 9.3-10.1 against 7.5-9.0 at 448.
 ONE_LAUNCH_TOKEN_HEADS = 512
+ONE_LAUNCH_K_BYTES = 160 << 10
 
 # Tiles of four query heads of 128 elements or more run two waves per SIMD; the policy splits
 # them into the ranges of four waves that one round of the chip holds, 2048 waves // (4 x tiles),
@@ -204,12 +207,14 @@ def policy_splits(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int
     simds = _one_split_waves(device, batch, num_q_heads, num_kv_heads, head_dim, block_size,
                              max_blocks, dtype)  # fmt: skip
     heads = min(num_q_heads // num_kv_heads, 4)  # per wave
-    if head_dim <= 128 and max_blocks * block_size * heads <= ONE_LAUNCH_TOKEN_HEADS:
+    tokens = max_blocks * block_size
+    if (head_dim <= 128 and tokens * heads <= ONE_LAUNCH_TOKEN_HEADS
+            and tokens * head_dim * dtype.itemsize <= ONE_LAUNCH_K_BYTES):  # fmt: skip
         return 1
     if heads == 4 and head_dim >= 128:
         tiles = batch * num_q_heads // heads
         ranges = min(IN_GROUP_MIN_WAVES // (2 * tiles), MAX_SPLITS, max_blocks)
-        return ranges if max_blocks * block_size * (ranges - 2) >= WIDE_RANGE_TOKENS else 1
+        return ranges if tokens * (ranges - 2) >= WIDE_RANGE_TOKENS else 1
     if simds >= IN_GROUP_MIN_WAVES // 2:
         return 1 if splits <= IN_GROUP_SPLITS else splits
     return max(splits, min(-(-2 * IN_GROUP_MIN_WAVES // max(simds, 1)), MAX_SPLITS, max_blocks))
