@@ -18,7 +18,8 @@ import torch.nn.functional as F
 
 from oracle import ref
 from tinyserve_amd.decode_step import (DecodeGraph, DecodeStep, KVPool, ModelShape, random_context_tables,
-                                       random_weights)  # fmt: skip
+                                       random_weights, rope_tables)  # fmt: skip
+from tinyserve_amd.hip_fused import rms_norm_rows
 from tinyserve_amd.step_inputs import Batch, DecodeInputs, PagedTable, build_batch, fill_decode_inputs
 
 pytestmark = pytest.mark.gpu
@@ -384,3 +385,18 @@ def test_config_5_bf16_rows_at_16_splits_against_library_projections() -> None:
     print(f"[config 5 bf16] rows/16 splits vs library/policy: logits max-abs {err:.3g} "
           f"(max |logit| {lib.float().abs().max().item():.3g})")
     torch.testing.assert_close(rows.float(), lib.float(), atol=CONFIG5_BF16_PATHS_ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_layers_one_by_one_give_the_step(dtype: torch.dtype) -> None:
+    # ``layer`` adds its last residual itself, where the step leaves it to the next norm: the
+    # same sums, bit for bit.
+    w, pool, _, inp = setup([3, 17, 40, 9, 1, 22, 5, 13], 8, dtype)
+    step = DecodeStep(TINY, w, pool, projections="library")
+    want = step.forward(inp)
+    cos, sin = rope_tables(TINY.head_dim, TINY.rope_theta, inp.positions)
+    x = w["model.embed_tokens.weight"][inp.token_ids]
+    for i in range(TINY.num_layers):
+        x = step.layer(i, x, cos, sin, inp.slots, lambda i, q: step._attention(i, q, inp))
+    h = rms_norm_rows(x, w["model.norm.weight"], TINY.rms_norm_eps)
+    assert torch.equal(F.linear(h, w["model.embed_tokens.weight"]).float(), want)

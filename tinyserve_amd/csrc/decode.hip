@@ -25,7 +25,8 @@
 //
 // Length pairs. A batch of at most 64 sequences that would get two-wave workgroups is
 // run as pairs instead: workgroup y takes the sequences ranked y and B - 1 - y by
-// length (longest with shortest), and its four waves take equal shares of the two
+// length (longest with shortest), and its waves (four, or eight where they stream or are
+// kLightWide) take equal shares of the two
 // sequences' blocks laid end to end (one wave may walk the end of one and the start of
 // the other). Every workgroup then has about the same work, so a batch of mixed
 // lengths does not wait on its longest sequences; equal lengths give the two-wave
@@ -43,7 +44,7 @@
 
 namespace ts {
 
-// Two register budgets. kHeavy: each lane streams 64 bytes of a head row per token, three
+// Register budgets. kHeavy: each lane streams 64 bytes of a head row per token, three
 // iterations in flight, one wave per SIMD (more than 256 VGPRs) -- for launches whose
 // waves all run in one round, where each wave must keep much in flight. kLight: 32 bytes
 // per lane, two in flight, two waves per SIMD -- for launches of several rounds, where
@@ -194,7 +195,7 @@ __device__ __forceinline__ void merge_token_lanes(TokenState<T, D, HT, LB>& st) 
   }
 }
 
-constexpr int kMaxWavesPerGroup = 4;  // heavy budget, and length pairs of cached launches
+constexpr int kMaxWavesPerGroup = 4;  // heavy budget; length pairs but streaming and wide ones
 constexpr int kMaxWavesLight = 8;     // light budget (two waves per SIMD)
 
 // LDS of a decode workgroup (dynamic, sized by the launch): NS state slots, each the

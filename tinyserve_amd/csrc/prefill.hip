@@ -33,8 +33,8 @@
 // workgroups and merged by a second kernel (the key cut, below).
 //
 // Three shapes: 8 waves with a 3-stage ring of 64-key tiles (one workgroup per CU, 98 KB
-// of LDS, two waves per SIMD) for large launches and prefix-hit chunks; for launches with
-// too few query tiles to fill the chip that way (one or two prompts), 8 waves over the
+// of LDS, two waves per SIMD) for large launches and prefix-hit chunks; for launches of few
+// query tiles and long walks (one or two prompts, chunks behind cached keys), 8 waves over the
 // queries of the 4-wave shape (64 x 2 heads) with the keys split in two: waves w and
 // w + 4 walk the lower and upper half of the key tiles (a 2-stage ring holding one tile
 // of each half, 128 KB) and merge their softmax states through LDS at the end, which
@@ -1021,10 +1021,8 @@ static int launch_prefill_mfma(const PrefillArgs& a, int Hkv, hipStream_t stream
   return launch_status();
 }
 
-// Query tiles of 32 * (W / HG) queries. The 8-wave shape is the faster one per unit of
-// work; the 4-wave shape halves the work per workgroup and fits two workgroups per CU,
-// which wins when the launch has fewer than two 8-wave workgroups per CU (e.g. one
-// 2048-token prompt: 128 workgroups of 8 waves).
+// Query tiles of 32 * (W / KP / HG) queries (KP: key parts), and the dispatch order. Which
+// shape a launch runs is prefill_shape's choice.
 template <typename T, int D, int W, int S, int BN, int OCC, int KP = 1>
 static int dispatch_hg_w(PrefillArgs& a, int Hkv, int max_q_len, int64_t n_rows, hipStream_t stream) {
   constexpr int WQ = W / KP;  // waves over the queries and heads
@@ -1128,13 +1126,14 @@ struct CutShape {
 // Whether a launch of these sizes may cut its keys, and how. max_keys: the block table's
 // width in keys, the most any sequence can have. The line: what a cut can save must exceed
 // the plan (~1 us), the merge launch (2 us empty, 9-10 us with 2-4 parts of 100 rows x 16
-// sequences) and the states' traffic. Measured at 16 q / 8 kv heads, D = 128, fp16 (cached
-// + new tokens, uncut -> cut, us): 16 x (500-5000 + 20-128) 114 -> 60, 1 x (8192 + 64)
-// 109 -> 26, 1 x (8192 + 512) 111 -> 55, 1 x (16000 + 32) 203 -> 29, 6 x (3000 + 128)
-// 79 -> 42, 24 x (0-6000 + 10-128) 144 -> 96, 8 x (2000 + 16) 32 -> 25; with equal lengths
-// on most of the chip the plan keeps items whole and costs 2-3 us (24 x (4096 + 128)
-// 136 -> 139). Below the line it lost: 4 x (1024 + 64) 21 -> 26, 4 x (8192 + 300) 115 ->
-// 125, 1 x (1500 + 256) 29 -> 33, 16 x (4096 + 64) 73 -> 75, 32 x (2048 + 128) 94 -> 99.
+// sequences) and the states' traffic. Measured at 16 q / 8 kv heads, D = 128, fp16 in graph
+// replay (cached + new tokens, uncut -> cut, us): 16 x (U[500, 5000] + U[20, 128]) 122 -> 78, 1 x
+// (8192 + 64) 110 -> 27, 1 x (8192 + 200) 109 -> 36, 1 x (8192 + 512) 113 -> 56, 1 x (16000 + 32)
+// 204 -> 30, 6 x (3000 + 128) 81 -> 43, 24 x (U[0, 6000] + U[10, 128]) 140 -> 107, 8 x (2000 + 16)
+// 33 -> 27; with equal lengths on most of the chip the plan keeps items whole (24 x (4096 + 128)
+// 152 -> 149-153). Below the line it lost, on other prefixes of these sizes: 4 x (1024 + 64) 21
+// -> 26, 4 x (8192 + 300) 115 -> 125, 1 x (1500 + 256) 29 -> 33, 16 x (4096 + 64) 73 -> 75, 32 x
+// (2048 + 128) 94 -> 99.
 static bool cut_shape(int R, int group, int Hkv, int D, int lbs, int max_q_len, int64_t max_keys, CutShape* c) {
   if (max_q_len > 512 || max_keys < 1024 || max_keys < 4 * static_cast<int64_t>(max_q_len)) return false;
   if ((1 << lbs) < kWave / (D / 8)) return false;  // scalar-id gather

@@ -72,8 +72,8 @@ IN_GROUP_MIN_WAVES = 1024
 # 6.9 against 7.8-8.4, fp32 256 tokens 7.7 against 8.2-8.6; 32 / 8 heads (four per wave) 128
 # tokens 7.8 against 9.1-10.1 but 208 tokens 10.8 against 9.2-11.0; called eagerly, 8.5-9.2
 # against 18-19 (two launches and three allocations of host time). The table's K per kv head is
-# bounded too: 32-bit rows of 128 elements at one head per wave are 7.5-8.2 us at 256 tokens
-# either way, 8.0-8.2 against 7.5-8.1 at 384 and 9.3-10.1 against 7.5-9.0 at 448.
+# bounded too: 32-bit rows of 128 elements at one head per wave take 6.7-7.0 against 7.6-8.4 at
+# 256 tokens, 8.0-8.2 against 7.5-8.1 at 384 and 9.3-10.1 against 7.5-9.0 at 448.
 ONE_LAUNCH_TOKEN_HEADS = 512
 ONE_LAUNCH_K_BYTES = 160 << 10
 
